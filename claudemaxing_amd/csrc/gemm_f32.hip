@@ -23,7 +23,12 @@ using cm::gemm::floatx16;
 using cm::gemm::KMajor;
 using cm::gemm::RowMajor;
 
-constexpr int kBM = 256, kBN = 192, kWM = 4, kWN = 2, kBK = 64, kStages = 2;
+// Tiles of 256 x 192 on 4 x 2 wavefronts of 64 x 96: with four of 128 x 96 long slices take the same
+// time and short ones more (131 x 1536 x 17920 31 us against 27). With the sum, one MI355X:
+// 1276 x 1536 x 17920 97 -> 82 us, x 8960 58 -> 51 us (the loads spread over the main loop and no
+// bounds test for the partial row of tiles, gemm_lds.h).
+constexpr int kBM = 256, kBN = 192, kWM = 4, kWN = 2, kBK = 64;
+constexpr int kSA = 3, kSB = 2;  // LDS stages of A and B: 144 KiB, one workgroup per CU
 constexpr int kThreads = kWM * kWN * cm::kWave;
 constexpr int kMaxSlices = 16;
 constexpr int kCUs = 256;
@@ -68,7 +73,7 @@ struct Pairs {
 template <bool KB>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int remap, float* ws,
                                                                int M, int N) {
-  __shared__ uint4 lds[kStages * (kBM + kBN) * (kBK / 8)];
+  __shared__ uint4 lds[(kSA * kBM + kSB * kBN) * (kBK / 8)];
   int tm, tn, s;
   cm::gemm::tile_of_block_2d((N + kBN - 1) / kBN, remap, tm, tn, s);
   const int q = s < p.slices0 ? 0 : 1, sq = q ? s - p.slices0 : s;
@@ -78,18 +83,18 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int rema
   EpiSlice epi{ws + static_cast<int64_t>(s) * M * N, M, N};
   if constexpr (KB) {
     if (q == 0) {
-      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kBK, kStages>(p.a[0], p.bk[0], k_begin, k_end, tm,
+      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[0], p.bk[0], k_begin, k_end, tm,
                                                            tn, epi, lds);
     } else {
-      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kBK, kStages>(p.a[1], p.bk[1], k_begin, k_end, tm,
+      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[1], p.bk[1], k_begin, k_end, tm,
                                                            tn, epi, lds);
     }
   } else {
     if (q == 0) {
-      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kBK, kStages>(p.a[0], p.b[0], k_begin, k_end, tm,
+      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[0], p.b[0], k_begin, k_end, tm,
                                                            tn, epi, lds);
     } else {
-      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kBK, kStages>(p.a[1], p.b[1], k_begin, k_end, tm,
+      cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[1], p.b[1], k_begin, k_end, tm,
                                                            tn, epi, lds);
     }
   }
@@ -130,7 +135,7 @@ struct Plan {
 };
 
 // Slices per pair in proportion to its K, so that tiles x slices is one round of workgroups
-// (one per CU: the LDS ring takes 112 KiB), in whole 64-column stages, at most 16 slices. At
+// (one per CU: the LDS ring takes 144 KiB), in whole 64-column stages, at most 16 slices. At
 // 40 tiles: 6 slices, 240 workgroups (10 slices in 1.6 rounds measured slower).
 Plan plan_for(int M, int N, int K0, int K1) {
   const int tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);

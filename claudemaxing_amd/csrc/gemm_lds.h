@@ -7,13 +7,15 @@
 // such instruction writes 64 consecutive 16-byte LDS slots (M0 base + 16 * lane); the XOR
 // swizzle of the LDS rows (swz()) is therefore applied on the global side: the lane that owns
 // LDS slot (row, physical chunk) fetches logical chunk physical ^ swz(row) of that row.
-// Chunks outside the operands (rows past the end, columns past k_len) are fetched from a
-// 16-byte zero block instead, so edge tiles need no separate path (hidden sizes are multiples
-// of 8, so a 16-byte chunk is either wholly inside or wholly outside).
+// Rows past the operands' end are fetched from the last valid row (they feed only outputs that are
+// never stored), so a tile at the edge costs nothing more; columns past k_len are fetched from a
+// 16-byte zero block (hidden sizes are multiples of 8, so a 16-byte chunk is either wholly inside
+// or wholly outside).
 //
-// The LDS holds a ring of S stages of BK (64 or 32) columns; stages kt + 1 .. kt + S - 1 are in
-// flight while stage kt is multiplied. One barrier per stage: after it every wavefront has finished reading stage
-// kt - 1 (so its buffer can be refilled) and every wavefront's loads of stage kt have landed.
+// The LDS holds a ring of SA stages of A and SB of B, each of 64 columns; the loads of stage
+// kt + SA - 1 of A and kt + SB - 1 of B are issued while stage kt is multiplied. One barrier per
+// stage: after it every wavefront has finished reading stage kt - 1 (so its buffers can be
+// refilled) and every wavefront's loads of stage kt have landed.
 //
 // An A-fragment transform FX may rescale each 8-element A fragment between the LDS read and the
 // MFMA (used by the LM head's gradient GEMM to turn stored e^{z - m} into probabilities). The
@@ -24,6 +26,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "gemm_nt.h"
@@ -95,12 +98,12 @@ template <int BK>
 using LdsRows = LdsTile<BK, false, 0>;
 
 // Direct loads of one ROWS x BK operand tile by NW wavefronts. Instruction i of a lane fills
-// LDS slot (i * NW + wave) * 64 + lane of the tile. Row-major: row row0 + i * kRowStep and (with
+// LDS slot (i * NW + wave) * 64 + lane of the tile: row-major, row row0 + i * kRowStep and (with
 // NW >= 2) the same swizzled column for every i, since kRowStep is a multiple of the swizzle's
-// period. Chunk-major: row row0 and column col0 + 8 i * kColStep. Either way a lane keeps one
-// byte offset from the stage origin, and instruction i adds i times a wave-uniform step; a
-// stage's origin is a wave-uniform pointer. Tiles that are wholly inside the operand take that
-// path; the others select the zero chunk per lane.
+// period; chunk-major, row row0 and column col0 + 8 i * kColStep. A lane keeps one byte offset
+// per instruction from the stage's origin, a wave-uniform pointer; rows past the operand's end
+// are already replaced in it (clamp_row), so a row edge takes no test in the loop (testing and
+// selecting per load cost 16 us of 93 where one tile row of five was partial: 1276 x 1536 x 17920).
 template <int ROWS, int NW, int BK, bool CM = false>
 struct DmaTile {
   using L = LdsTile<BK, CM, ROWS>;
@@ -111,43 +114,43 @@ struct DmaTile {
   static_assert(kPer * NW * kWave == kChunks, "tile chunks must split over the wavefronts");
   static_assert(CM || NW >= 2, "one swizzled column per lane needs a row step of 16 or more");
   static_assert(!CM || kColStep * ROWS == NW * kWave, "an instruction covers whole chunk columns");
-  uint32_t off0;      // byte offset of the lane's chunk of instruction 0 from the stage origin
-  uint32_t step;      // bytes between instructions (wave-uniform)
-  int row0, col0;     // tile row and column of the lane's chunk of instruction 0
+  // byte offset of the lane's chunk of instruction i from the stage origin (chunk-major:
+  // instruction 0's, the others a constant step apart)
+  uint32_t off[CM ? 1 : kPer];
+  int col0;  // tile column of the lane's chunk of instruction 0
 
+  // r0: the tile's first row (a valid one)
   template <class Src>
-  __device__ __forceinline__ void init(const Src& src, int wave, int lane) {
+  __device__ __forceinline__ void init(const Src& src, int r0, int wave, int lane) {
     const int c = wave * kWave + lane;
-    if (CM) {
-      row0 = c % ROWS;
-      col0 = (c / ROWS) * 8;
-      step = src.tile_offset(0, kColStep * 8);
-    } else {
-      row0 = c / L::kRC;
-      col0 = ((c % L::kRC) ^ L::swz(row0)) * 8;
-      step = src.tile_offset(kRowStep, 0);
-    }
-    off0 = src.tile_offset(row0, col0);
+    const int row0 = CM ? c % ROWS : c / L::kRC;
+    col0 = CM ? (c / ROWS) * 8 : ((c % L::kRC) ^ L::swz(row0)) * 8;
+#pragma unroll
+    for (int i = 0; i < (CM ? 1 : kPer); ++i)
+      off[i] = src.tile_offset(src.clamp_row(r0, row0 + i * kRowStep), col0);
+  }
+  template <class Src>
+  __device__ __forceinline__ uint32_t offset(int i) const {
+    if constexpr (CM) return off[0] + i * kColStep * Src::kChunkBytes;
+    else return off[i];
   }
 
-  // Instruction i of the stage whose origin is (r0, k0), for a tile known to lie wholly inside
-  // the operand: no bounds selection.
+  // Instruction i of the stage whose origin is (r0, k0), a stage wholly inside k_len.
   template <class Src>
   __device__ __forceinline__ void issue_inside(const Src& src, int r0, int k0, uint4* tile,
                                                int wave, int i) const {
     const char* base = reinterpret_cast<const char*>(src.at(r0, k0));
-    dma16(base + off0 + i * step, tile + (i * NW + wave) * kWave);
+    dma16(base + offset<Src>(i), tile + (i * NW + wave) * kWave);
   }
 
-  // Instruction i of the stage whose origin is (r0, k0); `inside` = the tile is wholly inside
-  // the operand (one wave-uniform test per stage).
+  // Instruction i of the stage whose origin is (r0, k0); `inside` = the stage lies wholly inside
+  // k_len (wave-uniform).
   template <class Src>
   __device__ __forceinline__ void issue(const Src& src, int r0, int k0, uint4* tile, int wave,
                                         int i, bool inside) const {
     const char* base = reinterpret_cast<const char*>(src.at(r0, k0));
-    const int row = row0 + i * kRowStep, col = col0 + i * kColStep * 8;
-    const bool ok = inside || (r0 + row < src.rows && src.col_ok(k0 + col));
-    const void* g = ok ? static_cast<const void*>(base + off0 + i * step)
+    const bool ok = inside || src.col_ok(k0 + col0 + i * kColStep * 8);
+    const void* g = ok ? static_cast<const void*>(base + offset<Src>(i))
                        : static_cast<const void*>(kZeroChunk);
     dma16(g, tile + (i * NW + wave) * kWave);
   }
@@ -159,8 +162,8 @@ struct DmaTile {
 // groups read rows k .. k + 3 (k a multiple of 4) at one 32-byte segment and the next, so with
 // this swizzle the 8 (row, segment) pieces a 32-lane half serves at once cover the 64 banks
 // exactly once. Instruction i of a lane fills slot c = (i NW + wave) 64 + lane of the tile: row
-// c / (BN / 8), physical slot c % (BN / 8); the slot positions differ per instruction, so the
-// lane keeps one byte offset per instruction.
+// c / (BN / 8), physical slot c % (BN / 8). As in DmaTile, a lane keeps one byte offset per
+// instruction; chunks past the operand's last n are read from its last whole chunk.
 template <int BN, int NW, int BK>
 struct DmaTileK {
   static constexpr int kSlotsRow = BN / 8;
@@ -170,18 +173,18 @@ struct DmaTileK {
   static_assert(BN % 64 == 0, "rows of whole groups of four 32-byte segments");
   static __device__ __forceinline__ int kswz(int k) { return ((k >> 1) & 1) * 2; }
   uint32_t off[kPer];  // byte offset of the lane's chunk of instruction i from the stage origin
-  int krow[kPer], ncol[kPer];
+  int krow[kPer];
 
   template <class Src>
-  __device__ __forceinline__ void init(const Src& src, int wave, int lane) {
+  __device__ __forceinline__ void init(const Src& src, int n0, int wave, int lane) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int c = (i * NW + wave) * kWave + lane;
       const int k = c / kSlotsRow, ps = c % kSlotsRow;
       const int ls = (((ps >> 1) ^ kswz(k)) << 1) | (ps & 1);  // logical slot of the row
       krow[i] = k;
-      ncol[i] = ls * 8;
-      off[i] = static_cast<uint32_t>((static_cast<int64_t>(k) * src.ld + ncol[i]) * 2);
+      const int n = min(ls * 8, (src.rows - n0 - 1) & ~7);
+      off[i] = static_cast<uint32_t>((static_cast<int64_t>(k) * src.ld + n) * 2);
     }
   }
   template <class Src>
@@ -194,7 +197,7 @@ struct DmaTileK {
   __device__ __forceinline__ void issue(const Src& src, int n0, int k0, uint4* tile, int wave,
                                         int i, bool inside) const {
     const char* base = reinterpret_cast<const char*>(src.at(n0, k0));
-    const bool ok = inside || (k0 + krow[i] < src.k_len && n0 + ncol[i] < src.rows);
+    const bool ok = inside || k0 + krow[i] < src.k_len;
     const void* g = ok ? static_cast<const void*>(base + off[i])
                        : static_cast<const void*>(kZeroChunk);
     dma16(g, tile + (i * NW + wave) * kWave);
@@ -246,38 +249,57 @@ struct ZeroStart {
   static __device__ __forceinline__ void started(floatx16 (&)[TM][TN]) {}
 };
 
-// Identity A-fragment transform with no per-stage data (the default FX of gemm_lds). An FX
-// provides bind(row) (the A row of the calling lane's fragment 0; fragment i is row + 32 i),
-// prefetch(k0) (register loads for the stage at column k0, issued one stage ahead),
-// advance() (the prefetched values become current) and apply(frag, i) on the A fragment of the
-// wavefront's tile row i.
+// Compile-time loop: f(std::integral_constant<int, 0>) .. f(std::integral_constant<int, N - 1>).
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Identity A-fragment transform (the default FX of gemm_lds). An FX may stage data of its own with
+// the A operand: kDma direct loads per wavefront and stage (issue(k0, slot), the last of A's loads
+// of the stage at column k0 into ring slot `slot`), fetch(slot) reads it back into registers at
+// the start of the stage, and apply(frag, i) transforms the A fragment of the wavefront's tile
+// row i.
 struct PlainA {
-  __device__ __forceinline__ void bind(int) {}
-  __device__ __forceinline__ void prefetch(int) {}
-  __device__ __forceinline__ void advance() {}
+  static constexpr int kDma = 0;
+  __device__ __forceinline__ void issue(int, int) const {}
+  __device__ __forceinline__ void fetch(int) {}
   __device__ __forceinline__ half8 apply(half8 f, int) const { return f; }
 };
 
-// Main loop, per stage kt: wait until stage kt has landed and this wavefront's fragment reads of
-// stage kt - 1 have returned, one barrier (stage kt visible; every wavefront is done with stage
-// kt - 1, whose buffer is refilled next), then five MFMA groups: the last substep of stage
-// kt - 1 (its fragments are already in registers, so these MFMAs cover the latency of the first
-// fragment reads of stage kt), then substeps 0 .. KS - 2 of stage kt, each after the reads of the
-// next substep's fragments. Each group issues its share of the loads of stage kt + S - 1 between
-// its two halves. Spreading the LDS-direct loads between MFMAs keeps the texture unit's queue
-// short, so a wavefront never stalls in issue with the matrix core idle (issued as one burst
-// after the barrier, the loads of a 256 x 256 x 64 stage held every wavefront for ~1000
-// cycles). sched_barrier pins that order.
-// Bounds handling of the operand loads (EDGE): kEdgeEither picks per workgroup (a second copy of
-// the main loop without bounds selection, taken when every stage lies inside both operands),
-// kEdgeAlways always selects, kEdgeNever never does (the caller guarantees every tile of the
-// launch lies inside: one loop, for kernels where two copies would not fit the registers).
+// Bounds handling of the operand loads' columns (EDGE): kEdgeEither picks per workgroup (a second
+// copy of the main loop without bounds selection, taken when every stage lies inside both
+// operands' k_len), kEdgeAlways always selects, kEdgeNever never does (the caller guarantees whole
+// stages: one loop, for kernels where two copies would not fit the registers).
 enum EdgeMode { kEdgeEither = 0, kEdgeAlways = 1, kEdgeNever = 2 };
 
-template <int BM, int BN, int WM, int WN, int BK, int S, class SrcA, class SrcB, class Epi,
+// Main loop, per stage kt: wait until stage kt has landed and this wavefront's fragment reads of
+// stage kt - 1 have returned, one barrier, then four groups of TM x TN MFMAs: the last 16-column
+// substep of stage kt - 1 (its fragments are already in registers, so these MFMAs cover the
+// latency of the first fragment reads of stage kt), then substeps 0 .. 2 of stage kt. The groups
+// are walked in slots of one MFMA: the first slots of a group also read one fragment of the next
+// substep each, and the stage's direct loads are spread evenly over the slots of all four groups
+// (of their first halves when both rings hold two stages), B's before A's when A's ring is the
+// deeper one. sched_barrier pins the order.
+//
+// What bounds it: the direct loads' issue. A CU takes one 1 KiB load instruction per ~16 cycles
+// (64 bytes per cycle, 57 measured), so several in a row from every wavefront at once hold the
+// wavefronts with the matrix cores idle; four in a row per group (an earlier form of this loop)
+// cost a quarter of the time: 8192 x 7680 x 8192 in 950 us with them, 715 us with the loads left
+// out, 922 us with the fragment reads left out. One load every four MFMAs needs a longer way
+// from issue to use than two stages give (the last load of a stage is then issued just before
+// the wait), hence the third stage of A; B, issued first, has half a stage and more. And a loop
+// without branches: the stages that load nothing, or only B, are separate copies. Together
+// 846 us, and 211 -> 176 us at 2048 x 1536 x 32768 in 4 slices with B k-major.
+template <int BM, int BN, int WM, int WN, int SA, int SB, class SrcA, class SrcB, class Epi,
           class FX = PlainA, int EDGE = kEdgeEither>
 __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_begin, int k_end,
                                          int tm, int tn, Epi& epi, uint4* lds, FX fx = FX()) {
+  constexpr int BK = 64;
   constexpr int NW = WM * WN;
   constexpr int WTM = BM / WM, WTN = BN / WN;
   constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -285,23 +307,29 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   using LB = LdsTile<BK, SrcB::kChunkMajor, BN>;
   constexpr int KS = BK / 16;  // MFMA substeps per stage
   static_assert(TM * 32 == WTM && TN * 32 == WTN, "wave tiles are multiples of 32");
-  static_assert(S >= 2, "at least a double buffer");
-  constexpr int kStage = (BM + BN) * LA::kRC;  // uint4 per stage
+  static_assert(SB >= 2 && (SA == SB || SA == SB + 1), "A's ring is B's or one stage deeper");
+  constexpr int kTileA = BM * LA::kRC, kTileB = BN * LB::kRC;  // uint4 per stage
   using TA = DmaTile<BM, NW, BK, SrcA::kChunkMajor>;
   static_assert(!SrcA::kKMajor, "a k-major operand is B");
   using TB = std::conditional_t<SrcB::kKMajor, DmaTileK<BN, NW, BK>,
                                 DmaTile<BN, NW, BK, SrcB::kChunkMajor>>;
-  constexpr int kDma = TA::kPer + TB::kPer;     // LDS-direct loads per lane per stage
-  constexpr int kPart = (kDma + KS - 1) / KS;   // of them issued per substep
-  constexpr int kHalf = (TM * TN) / 2;          // MFMAs before the loads of a substep
+  constexpr int kDmaA = TA::kPer + FX::kDma;  // direct loads per lane per stage
+  constexpr int kDmaB = TB::kPer;
+  constexpr int kDma = kDmaA + kDmaB;
+  constexpr int DA = SA - 1, DB = SB - 1;  // stages from issue to use
+  // loads of stage kt + 1 that may still be in flight when stage kt is needed
+  constexpr int kLate = DA > DB ? kDmaA : 0;
+  constexpr int NM = TM * TN, NR = TM + TN;  // MFMAs and fragments per substep
+  constexpr int kSlots = NM > NR ? NM : NR;
   const int m0 = tm * BM, n0 = tn * BN;
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int wm = wave / WN, wn = wave % WN;
+  uint4* const lds_b = lds + SA * kTileA;
   TA la;
   TB lb;
-  la.init(A, wave, lane);
-  lb.init(B, wave, lane);
+  la.init(A, m0, wave, lane);
+  lb.init(B, n0, wave, lane);
   epi.template prepare<TM, TN>(m0 + wm * WTM, n0 + wn * WTN, lane);
 
   // The epilogue's start() sets the accumulators (zero, or loads issued here so that they are
@@ -310,132 +338,125 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   epi.template start<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane);
 
   const int n_kt = (k_end - k_begin + BK - 1) / BK;
-  auto inside_a = [&](int kt) { return A.tile_inside(m0, BM, k_begin + kt * BK); };
-  auto inside_b = [&](int kt) { return B.tile_inside(n0, BN, k_begin + kt * BK); };
-  // Every stage of the workgroup's tiles lies inside both operands (the common case: the
-  // bounds tests are monotonic in the stage, so the last stage decides); the main loop then
-  // issues its loads with no bounds selection.
+  auto inside_a = [&](int kt) { return A.k_inside(k_begin + kt * BK); };
+  auto inside_b = [&](int kt) { return B.k_inside(k_begin + kt * BK); };
+  // Every stage lies inside both operands' columns (the common case: the bounds tests are
+  // monotonic in the stage, so the last stage decides); the main loop then issues its loads with
+  // no bounds selection.
   const bool all_inside = n_kt > 0 && inside_a(n_kt - 1) && inside_b(n_kt - 1);
-  // load instruction q (< kDma) of stage kt: A's instructions first, then B's
-  auto issue = [&](int kt, int q, bool in_a, bool in_b, auto edge) {
-    uint4* st = lds + (kt % S) * kStage;
+  auto load_a = [&](int kt, int i, auto edge) {
     const int k0 = k_begin + kt * BK;
-    if (q < TA::kPer) {
-      if constexpr (decltype(edge)::value) la.issue(A, m0, k0, st, wave, q, in_a);
-      else la.issue_inside(A, m0, k0, st, wave, q);
-    } else {
-      if constexpr (decltype(edge)::value) lb.issue(B, n0, k0, st + BM * LA::kRC, wave, q - TA::kPer, in_b);
-      else lb.issue_inside(B, n0, k0, st + BM * LA::kRC, wave, q - TA::kPer);
-    }
+    if (i >= TA::kPer) fx.issue(k0, kt % SA);
+    else if constexpr (decltype(edge)::value)
+      la.issue(A, m0, k0, lds + (kt % SA) * kTileA, wave, i, inside_a(kt));
+    else la.issue_inside(A, m0, k0, lds + (kt % SA) * kTileA, wave, i);
+  };
+  auto load_b = [&](int kt, int i, auto edge) {
+    const int k0 = k_begin + kt * BK;
+    if constexpr (decltype(edge)::value)
+      lb.issue(B, n0, k0, lds_b + (kt % SB) * kTileB, wave, i, inside_b(kt));
+    else lb.issue_inside(B, n0, k0, lds_b + (kt % SB) * kTileB, wave, i);
   };
   const int arow = wm * WTM + lane % 32, brow = wn * WTN + lane % 32;
   half8 af[2][TM], bf[2][TN];
-  auto read = [&](int kt, int ks, int buf) {
-    const uint4* As = lds + (kt % S) * kStage;
-    const uint4* Bs = As + BM * LA::kRC;
-    const int ch = ks * 2 + lane / 32;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) af[buf][i] = fx.apply(LA::frag(As, arow + i * 32, ch), i);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      if constexpr (SrcB::kKMajor) {
-        bf[buf][j] = frag_kmajor<BN>(Bs, wn * WTN + j * 32, ks, lane);
-      } else {
-        bf[buf][j] = LB::frag(Bs, brow + j * 32, ch);
-      }
+  // fragment r of substep ks, alternately of A and of B while both have one left: is_a(r) / its
+  // tile row or column
+  constexpr int kBoth = TM < TN ? TM : TN;
+  auto is_a = [](int r) { return r < 2 * kBoth ? r % 2 == 0 : TM > TN; };
+  auto index_of = [](int r) { return r < 2 * kBoth ? r / 2 : r - kBoth; };
+  auto read = [&](int kt, int ks, int buf, auto rc) {
+    constexpr int r = decltype(rc)::value;
+    const int ch = ks * 2 + lane / 32, x = index_of(r);
+    if (is_a(r)) {
+      af[buf][x] = LA::frag(lds + (kt % SA) * kTileA, arow + x * 32, ch);
+    } else {
+      const uint4* Bs = lds_b + (kt % SB) * kTileB;
+      if constexpr (SrcB::kKMajor) bf[buf][x] = frag_kmajor<BN>(Bs, wn * WTN + x * 32, ks, lane);
+      else bf[buf][x] = LB::frag(Bs, brow + x * 32, ch);
     }
   };
-  // Scheduling of a group "fragment reads of the next substep + first half of the MFMAs":
-  // one LDS read, one MFMA, alternately (measured 1.5% faster on the LM head than all reads
-  // first).
-  constexpr int kReads = TM + (SrcB::kKMajor ? 2 : 1) * TN;  // LDS reads per substep
-  auto interleave_reads = [] {
-#pragma unroll
-    for (int i = 0; i < (kReads > kHalf ? kReads : kHalf); ++i) {
-      if (i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-      if (i < kHalf) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);    // MFMA
-    }
-  };
-  auto mfma = [&](int b, int g0, int g1) {
-#pragma unroll
-    for (int g = g0; g < g1; ++g) {
-      const int i = g / TN, j = g % TN;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[b][i], bf[b][j], acc[i][j], 0, 0, 0);
-    }
+  auto mfma = [&](int b, int g) {
+    const int i = g / TN, j = g % TN;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[b][i], bf[b][j], acc[i][j], 0, 0, 0);
   };
 
-  // Prologue: stages 0 .. S - 2 in flight (the FX prefetch of stage 0 first).
-  fx.bind(m0 + wm * WTM + lane % 32);
-  if (n_kt > 0) fx.prefetch(k_begin);
+  // Prologue: the loads of the first stages, in the order in which the loop would issue them.
+  static_for<DA>([&](auto sc) {
+    constexpr int s = decltype(sc)::value;
+    if (s < DB && s < n_kt) {
 #pragma unroll
-  for (int s = 0; s < S - 1; ++s) {
-    if (s < n_kt) {
-      const bool ia = inside_a(s), ib = inside_b(s);
-#pragma unroll
-      for (int q = 0; q < kDma; ++q) issue(s, q, ia, ib, std::true_type{});
+      for (int i = 0; i < kDmaB; ++i) load_b(s, i, std::true_type{});
     }
-  }
+    if (s < n_kt) {
+#pragma unroll
+      for (int i = 0; i < kDmaA; ++i) load_a(s, i, std::true_type{});
+    }
+  });
 
   // Waits for the prologue's loads (the first stage and whatever start() issued).
   epi.template started<TM, TN>(acc);
 
-  // Stage kt. The last substep of stage kt - 1 is multiplied after the barrier of stage kt: its
-  // fragments are already in registers, so its MFMAs cover the latency of the first fragment
-  // reads of stage kt. Before the barrier each wavefront waits for its own reads (the buffer they
-  // read from is refilled after it). The bounds selection on the loads is compile-time (EDGE):
-  // with kEdgeEither a workgroup whose every stage lies inside both operands runs a copy of the
-  // loop without it. (Peeling the first stage and the load-free last stages as well, or two loop
-  // copies in the LM head's gradient GEMM, pushed it past 256 registers.)
-  static_assert(KS % 2 == 0, "substep buffers alternate within a stage");
-  auto run = [&](auto edge) {
-    for (int kt = 0; kt < n_kt; ++kt) {
-      if (kt + S - 2 < n_kt) {
-        wait_vmcnt<(S - 2) * kDma>();
-      } else {
-        wait_vmcnt<0>();
-      }
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): own fragment reads have landed
-      lds_barrier();
-      fx.advance();
-      if (kt + 1 < n_kt) fx.prefetch(k_begin + (kt + 1) * BK);
-      const int kl = kt + S - 1;
-      const bool load = kl < n_kt;
-      bool ia = true, ib = true;
-      if constexpr (decltype(edge)::value) {
-        ia = load && inside_a(kl);
-        ib = load && inside_b(kl);
-      }
-      read(kt, 0, 0);
-      if (kt > 0) {
-        mfma(1, 0, kHalf);
-        interleave_reads();
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (load) {
-#pragma unroll
-        for (int q = 0; q < kPart; ++q)
-          if (q < kDma) issue(kl, q, ia, ib, edge);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (kt > 0) mfma(1, kHalf, TM * TN);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks + 1 < KS; ++ks) {
-        const int b = ks & 1;
-        read(kt, ks + 1, b ^ 1);
-        mfma(b, 0, kHalf);
-        interleave_reads();
-        __builtin_amdgcn_sched_barrier(0);
-        if (load) {
-#pragma unroll
-          for (int q = (ks + 1) * kPart; q < (ks + 2) * kPart; ++q)
-            if (q < kDma) issue(kl, q, ia, ib, edge);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        mfma(b, kHalf, TM * TN);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+  // Direct load q of stage kt's slots: B's of stage kt + DB, then A's of stage kt + DA. LOADS: 2
+  // both, 1 B's alone, 0 none.
+  auto load = [&](int kt, int q, auto loads, auto edge) {
+    if (q < kDmaB) {
+      if constexpr (decltype(loads)::value >= 1) load_b(kt + DB, q, edge);
+    } else {
+      if constexpr (decltype(loads)::value == 2) load_a(kt + DA, q - kDmaB, edge);
     }
+  };
+  constexpr int kSpread = KS * NM / (DA > DB ? 1 : 2);  // MFMA slots the loads are spread over
+  // Group g of stage kt: reads the fragments of substep g (an FX is applied a few slots after its
+  // fragment's read), multiplies those of the substep before.
+  auto group = [&](int kt, auto gc, auto multiply, auto loads, auto edge) {
+    constexpr int g = decltype(gc)::value, buf = g & 1;
+    if constexpr (g == 0) fx.fetch(kt % SA);
+    static_for<kSlots>([&](auto mc) {
+      constexpr int m = decltype(mc)::value;
+      if constexpr (m < NR) read(kt, g, buf, mc);
+      if constexpr (m < NM && decltype(multiply)::value) mfma(buf ^ 1, m);
+      if constexpr (FX::kDma > 0) {
+        constexpr int kLag = kSlots - NR < 5 ? kSlots - NR : 5;
+        constexpr int r = m - kLag;
+        if constexpr (r >= 0 && r < NR)
+          if (is_a(r)) af[buf][index_of(r)] = fx.apply(af[buf][index_of(r)], index_of(r));
+      }
+      static_for<kDma>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        if constexpr ((2 * q + 1) * kSpread / (2 * kDma) == g * NM + m && m < NM)
+          load(kt, q, loads, edge);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  auto stage = [&](int kt, auto first, auto loads, auto edge) {
+    if (kLate > 0 && kt + 1 < n_kt) {
+      wait_vmcnt<kLate>();
+    } else {
+      wait_vmcnt<0>();
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): own fragment reads have landed
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    static_for<KS>([&](auto gc) {
+      constexpr bool kMul = decltype(gc)::value > 0 || !decltype(first)::value;
+      group(kt, gc, std::bool_constant<kMul>{}, loads, edge);
+    });
+  };
+  static_assert(KS % 2 == 0, "substep buffers alternate within a stage");
+  using Zero = std::integral_constant<int, 0>;
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  auto run = [&](auto edge) {
+    if (n_kt <= 0) return;
+    if (DA < n_kt) stage(0, std::true_type{}, Two{}, edge);
+    else if (DA > DB && DB < n_kt) stage(0, std::true_type{}, One{}, edge);
+    else stage(0, std::true_type{}, Zero{}, edge);
+    int kt = 1;
+    for (; kt + DA < n_kt; ++kt) stage(kt, std::false_type{}, Two{}, edge);
+    if constexpr (DA > DB)
+      for (; kt + DB < n_kt; ++kt) stage(kt, std::false_type{}, One{}, edge);
+    for (; kt < n_kt; ++kt) stage(kt, std::false_type{}, Zero{}, edge);
   };
   if constexpr (EDGE == kEdgeEither) {
     if (all_inside) {
@@ -447,7 +468,10 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
     (void)all_inside;
     run(std::bool_constant<EDGE == kEdgeAlways>{});
   }
-  if (n_kt > 0) mfma(1, 0, TM * TN);
+  if (n_kt > 0) {
+#pragma unroll
+    for (int g = 0; g < NM; ++g) mfma(1, g);
+  }
   epi.template apply<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane, lds);
 }
 

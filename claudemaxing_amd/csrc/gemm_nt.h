@@ -1,12 +1,11 @@
 // Operand layouts of the fp16 "NT" GEMMs on the gfx950 matrix cores (C[m][n] = sum_k A[m][k]
 // B[n][k], both operands K-contiguous), the MFMA register types, and the workgroup -> tile map.
 //   RowMajor  element (r, k) at p[r * ld + k];
-//   Blocked64 element (r, k) at p[((k / 64) * rows + r) * 64 + k % 64], i.e. 64-column panels,
-//             so a (rows x 64) tile of one panel is a single contiguous span. Panels are padded
-//             to 64 columns (the padding must hold finite values; the LM head keeps zeros there).
 //   Tiled32   32-row x 64-column blocks of 8-column chunks (below);
 //   KMajor    the operand stored transposed, [K][N] with N contiguous (below).
-// The main loop that consumes them is in gemm_lds.h.
+// The main loop that consumes them is in gemm_lds.h. Of a tile that reaches past the operand's last
+// row, the rows outside are read from its last valid row: they feed only outputs that are never
+// stored. Columns past k_len must come as zeros (k_inside says whether a stage has any).
 #pragma once
 
 #include "common.h"
@@ -30,33 +29,13 @@ struct RowMajor {
   __device__ __forceinline__ const _Float16* at(int r, int k) const {
     return p + static_cast<int64_t>(r) * ld + k;
   }
-  __device__ __forceinline__ bool tile_inside(int r0, int n_rows, int k0) const {
-    return r0 + n_rows <= rows && k0 + kBK <= k_len;
-  }
+  __device__ __forceinline__ bool k_inside(int k0) const { return k0 + kBK <= k_len; }
   __device__ __forceinline__ bool col_ok(int k) const { return k < k_len; }
+  // the row of a tile at r0 that stands in for its row r (valid rows for themselves)
+  __device__ __forceinline__ int clamp_row(int r0, int r) const { return min(r, rows - 1 - r0); }
   // bytes from element (r0, k0) to (r0 + r, k0 + k) of a tile (k < 64)
   __device__ __forceinline__ uint32_t tile_offset(int r, int k) const {
     return static_cast<uint32_t>((static_cast<int64_t>(r) * ld + k) * 2);
-  }
-};
-
-struct Blocked64 {
-  static constexpr bool kChunkMajor = false;
-  static constexpr bool kKMajor = false;
-  const _Float16* p;
-  int rows;   // valid rows (= rows of a panel)
-  int k_len;  // columns, padded panels beyond it hold finite values
-  __device__ __forceinline__ const _Float16* at(int r, int k) const {
-    return p + ((static_cast<int64_t>(k / kBK) * rows + r) * kBK + k % kBK);
-  }
-  __device__ __forceinline__ bool tile_inside(int r0, int n_rows, int k0) const {
-    return r0 + n_rows <= rows && k0 < k_len;
-  }
-  // the panel holding k exists (padding columns are read as stored)
-  __device__ __forceinline__ bool col_ok(int k) const { return (k / kBK) * kBK < k_len; }
-  // bytes from element (r0, k0) to (r0 + r, k0 + k) of a tile (k0 a multiple of 64, k < 64)
-  __device__ __forceinline__ uint32_t tile_offset(int r, int k) const {
-    return static_cast<uint32_t>((r * kBK + k) * 2);
   }
 };
 
@@ -66,10 +45,11 @@ struct Blocked64 {
 // chunks of 32 consecutive rows at one 8-column position are one 512-byte span, so a producer
 // whose lanes hold consecutive rows (the LM head's logits epilogue: one token per lane) writes
 // whole spans straight from registers, while a GEMM stage's 8-row x 64-column slices stay inside
-// one block. As with Blocked64, the columns up to the end of the last 64-column panel must hold
-// finite values.
+// one block. The columns up to the end of the last 64-column panel must hold finite
+// values, and the rows up to the end of the last tile must exist (their values are not used).
 struct Tiled32 {
   static constexpr bool kChunkMajor = true;
+  static constexpr int kChunkBytes = 512;  // between a row's neighbouring 8-column chunks
   static constexpr bool kKMajor = false;
   const _Float16* p;
   int rows;        // valid rows
@@ -81,14 +61,13 @@ struct Tiled32 {
   __device__ __forceinline__ const _Float16* at(int r, int k) const {
     return p + index(r, k, row_blocks);
   }
-  __device__ __forceinline__ bool tile_inside(int r0, int n_rows, int k0) const {
-    return r0 + n_rows <= rows && k0 < k_len;
-  }
+  __device__ __forceinline__ bool k_inside(int k0) const { return k0 < k_len; }
   __device__ __forceinline__ bool col_ok(int k) const { return (k / kBK) * kBK < k_len; }
+  __device__ __forceinline__ int clamp_row(int, int r) const { return r; }
   // bytes from element (r0, k0) to (r0 + r, k0 + k) of a tile (r0 a multiple of 32, k0 of 64,
   // k < 64 a multiple of 8)
   __device__ __forceinline__ uint32_t tile_offset(int r, int k) const {
-    return static_cast<uint32_t>(((r / 32) * 8 + k / 8) * 512 + (r % 32) * 16);
+    return static_cast<uint32_t>(((r / 32) * 8 + k / 8) * kChunkBytes + (r % 32) * 16);
   }
 };
 
@@ -107,26 +86,13 @@ struct KMajor {
   __device__ __forceinline__ const _Float16* at(int n, int k) const {
     return p + static_cast<int64_t>(k) * ld + n;
   }
-  __device__ __forceinline__ bool tile_inside(int n0, int n_rows, int k0) const {
-    return n0 + n_rows <= rows && k0 + kBK <= k_len;
-  }
+  __device__ __forceinline__ bool k_inside(int k0) const { return k0 + kBK <= k_len; }
 };
 
-// Workgroup -> (tile_m, tile_n), tile_n fastest. With remap (grid a multiple of 8), logical tile
-// ids are laid out so that consecutive ones run on the same XCD (hardware dispatches workgroup
-// ids round-robin over the 8 XCDs), so workgroups that share operand tiles share an L2.
-__device__ __forceinline__ void tile_of_block(int tiles_n, int remap, int& tm, int& tn) {
-  int bid = blockIdx.x;
-  if (remap) {
-    const int per = gridDim.x / 8;
-    bid = (bid % 8) * per + bid / 8;
-  }
-  tm = bid / tiles_n;
-  tn = bid % tiles_n;
-}
-
-// The same for block `bid` of `count` blocks of one role inside a larger grid (the caller keeps
-// bid % 8 equal to the block's XCD). remap requires count % 8 == 0.
+// Workgroup -> (tile_m, tile_n), tile_n fastest, for block `bid` of `count` blocks. With remap
+// (count % 8 == 0), logical tile ids are laid out so that consecutive ones run on the same XCD
+// (hardware dispatches workgroup ids round-robin over the 8 XCDs), so workgroups that share operand
+// tiles share an L2.
 __device__ __forceinline__ void tile_of(int bid, int count, int tiles_n, int remap, int& tm,
                                         int& tn) {
   if (remap) bid = (bid % 8) * (count / 8) + bid / 8;

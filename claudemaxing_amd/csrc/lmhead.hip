@@ -58,23 +58,32 @@ constexpr int kMaxSplit = 32;      // K-slices of the gradient GEMM (small batch
 constexpr int kFinalUnrolled = 8;  // K4 slice counts with their own instantiation
 constexpr int kRowsPerBlock = 4;  // K2: token rows (one wavefront each) per workgroup
 
-// Tile configurations: BM, BN, wavefront grid WM x WN, stage depth BK, LDS ring stages, and the
-// minimum wavefronts per SIMD for __launch_bounds__ (which caps the registers per wavefront:
-// 2 gives 256, 1 gives 512).
-constexpr int kBM1 = 256, kBN1 = 256, kWM1 = 2, kWN1 = 4, kBK1 = 64, kST1 = 2, kOcc1 = 2;
+// Tile configurations: BM, BN, wavefront grid WM x WN, LDS ring stages of A and of B (64 columns
+// each), and the minimum wavefronts per SIMD for __launch_bounds__ (which caps the registers per
+// wavefront: 2 gives 256, 1 gives 512). K1 stays at eight wavefronts: its epilogue is vector
+// arithmetic on the accumulators, which four wavefronts of 128 x 128 would hold in accumulation
+// registers and copy out one by one (961 us for the call without the gradient against 1011 us on
+// four, N = 2048; 989 us with the ring of two stages each).
+constexpr int kBM1 = 256, kBN1 = 256, kWM1 = 2, kWN1 = 4, kSA1 = 3, kSB1 = 2, kOcc1 = 2;
 constexpr int kThreads1 = kWM1 * kWN1 * cm::kWave;
 // K3's tile configurations, one per kind of hidden size (the tile's columns): 256 tokens x 192
-// hidden units on 4 x 2 wavefronts of 64 x 96 where the hidden size is a multiple of 192
-// (Qwen2.5-1.5B's 1536: 8 tiles per 256 tokens, no partial tile), else 256 x 256 on 2 x 4 of
-// 128 x 64 where it is a multiple of 256 (2048, 3584, 5120, 8192), else the first.
-template <int BM, int BN, int WM, int WN, int BK, int ST, int OCC>
+// hidden units on 2 x 2 wavefronts of 128 x 96 where the hidden size is a multiple of 192
+// (Qwen2.5-1.5B's 1536: 8 tiles per 256 tokens, no partial tile), else 256 x 256 on 4 x 2 of
+// 64 x 128 where it is a multiple of 256 (2048, 3584, 5120, 8192), else the first. The square
+// tile's rings stay at two stages of each operand: a third stage of E would leave no LDS for the
+// scales. Whole calls, one MI355X: N = 2048 at 1536 2102 -> 1950 us (four or eight wavefronts
+// alike), at 2048 2661 -> 2558 us (2575 on 2 x 4 wavefronts, 3181 on four, which spill, 3125 on
+// 256 x 192 tiles with a partial last one); 131 tokens at 1536 325 -> 292 us.
+template <int BM, int BN, int WM, int WN, int SA, int SB, int OCC>
 struct K3Cfg {
-  static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kBK = BK, kST = ST, kOcc = OCC;
+  static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kSA = SA, kSB = SB, kOcc = OCC;
   static constexpr int kThreads = WM * WN * cm::kWave;
-  static constexpr int kLds = ST * (BM + BN) * (BK / 8);  // uint4 of the LDS ring
+  static constexpr int kRing = (SA * BM + SB * BN) * 8;  // uint4 of the operands' LDS rings
+  // and of the scales': the fp32 scales of the tile's BM = 256 token rows per stage of E
+  static constexpr int kLds = kRing + SA * cm::kWave;
 };
-using K3Tall = K3Cfg<256, 192, 4, 2, 64, 2, 2>;
-using K3Square = K3Cfg<256, 256, 2, 4, 64, 2, 2>;
+using K3Tall = K3Cfg<256, 192, 2, 2, 3, 2, 1>;
+using K3Square = K3Cfg<256, 256, 4, 2, 2, 2, 2>;
 __host__ __device__ constexpr bool k3_square(int hidden) {
   return hidden % 192 != 0 && hidden % 256 == 0;
 }
@@ -335,28 +344,29 @@ struct EpiGrad {
 
 // K3's A-fragment transform: E (fp16 e^{z - m_g}) times the (token, group) scale
 // s_g = e^{m_g - lse} * 1024 (0 for unlabelled tokens) gives P16 = e^{z - lse} * 1024. The
-// scales of the next stage are loaded one stage ahead; each A fragment (8 columns of one token,
-// all inside one group) then costs four packed fp16 multiplies.
+// scales travel with E's tiles: one load instruction per stage and wavefront brings those of the
+// tile's 256 token rows straight into the LDS (the group of a stage is one row of the scale array,
+// whose token rows are padded to whole tiles; every wavefront writes the same bytes to the same
+// slots, so none depends on another's), and the main loop's waits count it like the operand
+// loads; loads into registers would make the compiler wait for every load in flight before their
+// use. Each A fragment (8 columns of one token, all inside one group) then costs four packed fp16
+// multiplies.
 template <int TM>
 struct ScaleP {
-  const float* scale;  // [groups][n_tok]
-  int n_tok;
-  int row = 0;
-  float nxt[TM];
+  static constexpr int kDma = 1;
+  const float* scale;  // [groups][row_stride], at the workgroup's first token row
+  int64_t row_stride;
+  uint4* lds;          // 64 slots per ring slot
+  int lane, row;       // row: the lane's token row of the tile in its wavefront's fragment 0
   _Float16 cur[TM];
 
-  __device__ __forceinline__ void bind(int r) { row = r; }
-  __device__ __forceinline__ void prefetch(int k0) {
-    const float* s = scale + static_cast<int64_t>(k0 / kGroup) * n_tok;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int r = row + 32 * i;
-      nxt[i] = r < n_tok ? s[r] : 0.0f;
-    }
+  __device__ __forceinline__ void issue(int k0, int slot) const {
+    cm::gemm::dma16(scale + (k0 / kGroup) * row_stride + lane * 4, lds + slot * cm::kWave);
   }
-  __device__ __forceinline__ void advance() {
+  __device__ __forceinline__ void fetch(int slot) {
+    const float* s = reinterpret_cast<const float*>(lds + slot * cm::kWave) + row;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) cur[i] = static_cast<_Float16>(nxt[i]);
+    for (int i = 0; i < TM; ++i) cur[i] = static_cast<_Float16>(s[32 * i]);
   }
   __device__ __forceinline__ half8 apply(half8 f, int i) const { return f * cur[i]; }
 };
@@ -386,16 +396,17 @@ struct K3Job {
   int n_tok, hidden;
   const float* factor;
   int first;
-  const float* scale;
+  const float* scale;  // [groups][scale_rows]
+  int64_t scale_rows;
 };
 
-constexpr int kLds1 = kST1 * (kBM1 + kBN1) * (kBK1 / 8);  // uint4 of K1's LDS ring
+constexpr int kLds1 = (kSA1 * kBM1 + kSB1 * kBN1) * 8;  // uint4 of K1's LDS ring
 
 __device__ __forceinline__ void k1_block(const K1Job& j, int bid, uint4* lds) {
   int tm, tn;
   cm::gemm::tile_of(bid, j.count, (j.B.rows + kBN1 - 1) / kBN1, j.remap, tm, tn);
   EpiProbs epi = j.epi;
-  cm::gemm::gemm_lds<kBM1, kBN1, kWM1, kWN1, kBK1, kST1>(j.A, j.B, 0, j.A.k_len, tm, tn, epi, lds);
+  cm::gemm::gemm_lds<kBM1, kBN1, kWM1, kWN1, kSA1, kSB1>(j.A, j.B, 0, j.A.k_len, tm, tn, epi, lds);
 }
 
 template <class CFG, int EDGE>
@@ -409,8 +420,16 @@ __device__ __forceinline__ void k3_block(const K3Job& j, int bid, uint4* lds) {
   const int k_end = max(k_begin, min(j.A.k_len, k_begin + j.k_slice));
   EpiGrad epi{j.out.g[s], j.n_tok, j.hidden, j.factor, j.first, {}};  // f: start()
   using FX = ScaleP<CFG::kBM / CFG::kWM / 32>;
-  FX xp{j.scale, j.n_tok, 0, {}, {}};  // nxt / cur are filled by prefetch
-  cm::gemm::gemm_lds<CFG::kBM, CFG::kBN, CFG::kWM, CFG::kWN, CFG::kBK, CFG::kST, Tiled32, KMajor,
+  static_assert(CFG::kBM == 4 * cm::kWave, "a wavefront's load covers the tile's token rows");
+  const int lane = threadIdx.x % cm::kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / cm::kWave);
+  FX xp{j.scale + tm * CFG::kBM,
+        j.scale_rows,
+        lds + CFG::kRing,
+        lane,
+        wave / CFG::kWN * (CFG::kBM / CFG::kWM) + lane % 32,
+        {}};  // cur: fetch()
+  cm::gemm::gemm_lds<CFG::kBM, CFG::kBN, CFG::kWM, CFG::kWN, CFG::kSA, CFG::kSB, Tiled32, KMajor,
                      EpiGrad, FX, EDGE>(j.A, j.B, k_begin, k_end, tm, tn, epi, lds, xp);
 }
 
@@ -421,8 +440,7 @@ __global__ __launch_bounds__(kThreads1, kOcc1) void lmh_gemm1(K1Job j) {
   k1_block(j, static_cast<int>(blockIdx.x), lds);
 }
 
-// EDGE: cm::gemm::kEdgeNever when every output tile lies inside G (n_tok a multiple of the
-// tile's rows, hidden of its columns; the contraction runs over whole 64-column panels), else
+// EDGE: cm::gemm::kEdgeNever when the contraction runs over whole 64-column panels, else
 // kEdgeAlways. One loop copy per kernel: two in one did not fit the registers.
 template <class CFG, int EDGE>
 __global__ __launch_bounds__(CFG::kThreads, CFG::kOcc) void lmh_gemm3(K3Job j) {
@@ -503,7 +521,7 @@ __device__ __forceinline__ OffState wave_merge_off(OffState s) {
 }
 
 // K2: merge the chunk's partials into the running state; the factor; with a scale array, the
-// group scales s_g = e^{m_g - lse} * 1024 of labelled tokens ([groups][n_tok], 0 otherwise),
+// group scales s_g = e^{m_g - lse} * 1024 of labelled tokens ([groups][scale_rows], 0 otherwise),
 // and the label's own entry of E set to 0 when the label falls in this chunk: the label's
 // coefficient p_t - 1 is applied by K4 in fp32, so its near-1 probability never enters the
 // fp32 accumulators (a ~1024 W_t term there would cancel against -1024 W_t only at the end,
@@ -517,8 +535,8 @@ template <int SLOTS>
 __global__ __launch_bounds__(kRowsPerBlock * cm::kWave) void lmh_rows_kernel(
     const Partial* __restrict__ part, int n_groups, RowState rs,
     const int64_t* __restrict__ target, int n_tok, int64_t c0, int n_voc, int first,
-    float* __restrict__ scale, _Float16* __restrict__ e16, const _Float16* __restrict__ label_z,
-    int row_blocks) {
+    float* __restrict__ scale, int64_t scale_rows, _Float16* __restrict__ e16,
+    const _Float16* __restrict__ label_z, int row_blocks) {
   const int lane = threadIdx.x % cm::kWave;
   const int row = blockIdx.x * kRowsPerBlock + static_cast<int>(threadIdx.x / cm::kWave);
   if (row >= n_tok) return;  // the whole wavefront
@@ -593,7 +611,7 @@ __global__ __launch_bounds__(kRowsPerBlock * cm::kWave) void lmh_rows_kernel(
   for (int i = 0; i < SLOTS; ++i) {
     const int g = lane + i * cm::kWave;
     if (g < n_valid)
-      scale[static_cast<int64_t>(g) * n_tok + row] =
+      scale[g * scale_rows + row] =
           labelled ? cm::exp_f(p[i].max - lse_now) * kPScale : 0.0f;
   }
   if (lane == 0 && g_label >= 0)
@@ -827,7 +845,7 @@ Layout layout(int64_t n_rows, int64_t vocab, int hidden, int64_t chunk, bool wan
   L.off_labz = off;
   off += round_up(n_rows * 2 * kEpiRows * 2, 256);
   L.off_scale = off;
-  off += round_up(n_rows * L.n_groups * 4, 256);
+  off += e_rows(n_rows) * L.n_groups * 4;  // padded to K3's tiles, as E
   L.off_g = off;
   off += (L.n_split - 1) * round_up(n_rows * hidden * 4, 256);
   L.total = off;
@@ -912,15 +930,16 @@ int run_lmhead(const void* hidden, int64_t ld_h, const void* weight, int64_t ld_
     const int64_t c0 = c0_of(c);
     _Float16* e = e16_of(c);
     const int rb = e_row_blocks(n_tok);
+    const int64_t sr = e_rows(n_tok);
     if (L.n_groups <= cm::kWave) {
       hipLaunchKernelGGL(lmh_rows_kernel<1>, grid, block, 0, s, part, ng, rs, target, n_tok, c0,
-                         nv, fi, scale, e, label_z, rb);
+                         nv, fi, scale, sr, e, label_z, rb);
     } else if (L.n_groups <= 4 * cm::kWave) {
       hipLaunchKernelGGL(lmh_rows_kernel<4>, grid, block, 0, s, part, ng, rs, target, n_tok, c0,
-                         nv, fi, scale, e, label_z, rb);
+                         nv, fi, scale, sr, e, label_z, rb);
     } else {
       hipLaunchKernelGGL(lmh_rows_kernel<kMaxRowSlots>, grid, block, 0, s, part, ng, rs, target,
-                         n_tok, c0, nv, fi, scale, e, label_z, rb);
+                         n_tok, c0, nv, fi, scale, sr, e, label_z, rb);
     }
     return cm::launch_status();
   };
@@ -944,7 +963,8 @@ int run_lmhead(const void* hidden, int64_t ld_h, const void* weight, int64_t ld_
             hidden_size,
             rs.factor,
             c == 0 ? 1 : 0,
-            scale};
+            scale,
+            e_rows(n_tok)};
     return j;
   };
 
@@ -960,9 +980,9 @@ int run_lmhead(const void* hidden, int64_t ld_h, const void* weight, int64_t ld_
     const K3Job j3 = k3_job(c);
     auto launch3 = [&](auto cfg) {
       using CFG = decltype(cfg);
-      // E's rows are padded to whole tiles (kERowAlign), so only the hidden size and the
-      // chunk's columns decide whether every load lies inside its operand
-      if (hidden_size % CFG::kBN == 0 && j3.A.k_len % CFG::kBK == 0) {
+      // edges of the tokens and of the hidden size cost the loads nothing (gemm_lds.h): only the
+      // chunk's columns decide whether every stage is whole
+      if (j3.A.k_len % kPanel == 0) {
         hipLaunchKernelGGL((lmh_gemm3<CFG, cm::gemm::kEdgeNever>), dim3(j3.count),
                            dim3(CFG::kThreads), 0, s, j3);
       } else {

@@ -341,8 +341,8 @@ __global__ __launch_bounds__(kThreads, 2) void nf4_gemm_kernel(const Args args) 
   auto issue_b = [&](int kt, uint4* st) {
     const int wi = stage_w(kt), kc = stage_k(kt, wi);
     const RowMajor src = token_src(wi);
-    lb.init(src, wave, lane);
-    const bool inside = src.tile_inside(m0, BN, kc);
+    lb.init(src, m0, wave, lane);
+    const bool inside = src.k_inside(kc);
 #pragma unroll
     for (int q = 0; q < TB::kPer; ++q) lb.issue(src, m0, kc, st + BM * kRC, wave, q, inside);
   };
@@ -630,8 +630,8 @@ __global__ __launch_bounds__(kWsThreads, 1) void nf4_gemm_v3(const Args args) {
         src.k_len = cols;
       }
       src.rows = args.m;
-      lb.init(src, pw, lane);
-      const bool inside = src.tile_inside(m0, BN, kc);
+      lb.init(src, m0, pw, lane);
+      const bool inside = src.k_inside(kc);
 #pragma unroll
       for (int q = 0; q < TB::kPer; ++q) lb.issue(src, m0, kc, slot, pw, q, inside);
       const char* pk = reinterpret_cast<const char*>(w.packed);

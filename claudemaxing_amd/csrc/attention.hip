@@ -12,15 +12,16 @@
 // Layout. Rows are laid out "row-aligned" in a padded position space: row r starts at position
 // pstart[r] = sum over earlier rows of round_up(len, 64), so every 64-token block of a row
 // starts 64-aligned and the MFMA operand tiles are whole 16-byte chunks. A relayout pass writes
-// fp16 copies of the operands in that space, zero in the pad slots:
-//   natural    X16[head][pos][d]                      (d contiguous)
-//   transposed XT16[head][d][pos] with the positions of every 16-group stored in the order
-//              0-3, 8-11, 4-7, 12-15 (bits 2 and 3 of the position swapped).
-// The order is the one in which a lane of a 32x32 MFMA accumulator holds its 16 rows: lane l
-// holds rows (e/4)*8 + (l/32)*4 + e%4, so accumulator elements 8j..8j+7 are, in that order, the 8
-// operand slots of k-step j for half l/32. A probability tile computed as an accumulator thus
-// feeds the next MFMA straight from registers, against a transposed operand tile read as one
-// 16-byte chunk per lane.
+// fp16 copies X16[head][pos][d] (d contiguous) of the operands in that space, zero in the pad
+// slots. An MFMA operand that contracts over positions (V in O^T += V^T P^T, Q, dO and K in the
+// backward) is read from the same tiles with transposing LDS reads (frag_t), four positions of one
+// d per 8-byte read. Lane l of a 32x32 MFMA accumulator holds rows (e/4)*8 + (l/32)*4 + e%4, so
+// accumulator elements 8j..8j+7 are the 8 operand slots of k-step j for half l/32 once the other
+// operand's slots are taken in the same order (positions 0-3 and 8-11 of the 16 for the first half,
+// 4-7 and 12-15 for the second), which two transposing reads give: a probability tile computed as an
+// accumulator feeds the next MFMA straight from registers. (Separate transposed copies, an earlier
+// form, doubled the backward's tiles: one workgroup per CU instead of two, and the copies' own
+// traffic.)
 //
 // The row bounds are a device-resident image (Rows, written by cm_attn_rows_image on the host and
 // copied to the device by the caller) and the grids are sized for a capacity of padded positions
@@ -51,7 +52,6 @@ constexpr int kD = 128;       // head dimension
 constexpr int kBlk = 64;      // tokens per block (rows are padded to multiples of it)
 constexpr int kMaxRows = 128; // rows of one packed batch
 constexpr int kThreads = 256; // two pairs of wavefronts of 32 queries (or keys) each
-constexpr int kPairThreads = 128;
 
 struct Rows {
   int start[kMaxRows + 1];   // first real token of row r; start[n] = number of tokens
@@ -132,11 +132,6 @@ __device__ __forceinline__ Where locate(const Rows& rows, int b, int n_tokens, i
 // it keeps the natural order.
 __device__ __forceinline__ int heavy_first_query_block() {
   return static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
-}
-
-// Stored slot of position p inside its 16-group (an involution: bits 2 and 3 swapped).
-__device__ __forceinline__ int perm16(int p) {
-  return (p & ~12) | ((p & 4) << 1) | ((p & 8) >> 1);
 }
 
 __device__ __forceinline__ floatx16 mfma(half8 a, half8 b, floatx16 c) {
@@ -220,34 +215,49 @@ __device__ __forceinline__ float rot_plus(float x, float p, float cs, float sn) 
 }
 
 // LDS tiles filled by global_load_lds_dwordx4 (64 lanes x 16 bytes into 64 consecutive slots).
-// A tile has ROWS rows of CH 16-byte chunks; the chunk of (row, logical c) is stored at
-// physical chunk c ^ swz(row), chosen so that a fragment read (16 consecutive rows at one
-// logical chunk per 16 lanes) hits 16 distinct bank groups:
-//   CH = 16 (256-byte rows): row & 15;  CH = 8: (row >> 1) & 7;  CH = 4: (row >> 2) & 3.
-template <int CH>
-__device__ __forceinline__ int swz(int row) {
-  return CH == 16 ? (row & 15) : CH == 8 ? ((row >> 1) & 7) : ((row >> 2) & 3);
-}
+// A tile has rows of kCh 16-byte chunks (the 128 values of d of one position); the chunk of (row,
+// logical c) is stored at physical chunk c ^ swz(row). A fragment read (frag) takes 16 consecutive
+// rows at one logical chunk per 16 lanes: 16 distinct swz, so 16 distinct bank groups. A transposing
+// read (frag_t) takes 4 consecutive rows at 4 consecutive chunks per 32 lanes: the row's two low bits
+// choose the quarter of the 256-byte row, so it covers the 64 banks once too.
+constexpr int kCh = kD / 8;
+__device__ __forceinline__ int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
-template <int CH>
 __device__ __forceinline__ half8 frag(const uint4* tile, int row, int c) {
-  return __builtin_bit_cast(half8, tile[row * CH + (c ^ swz<CH>(row))]);
+  return __builtin_bit_cast(half8, tile[row * kCh + (c ^ swz(row))]);
 }
 
-// Issue this thread's loads of a ROWS x CH tile whose row i starts at src + i * row_bytes; the
-// two wavefronts of a pair (wave = 0, 1 within the pair) load a tile together.
-template <int ROWS, int CH>
-__device__ __forceinline__ void load_tile(uint4* tile, const void* src, int64_t row_bytes,
-                                          int wave, int lane) {
-  constexpr int kNW = kPairThreads / cm::kWave;
-  constexpr int kPer = ROWS * CH / kPairThreads;
-  static_assert(kPer * kPairThreads == ROWS * CH, "tile chunks split over the pair");
+// The operand of k-step j (positions 16 j .. 16 j + 15 of the tile, in the accumulators' order) whose
+// rows are d = d0 .. d0 + 31: lane l gets d = d0 + l % 32 at positions 16 j + 4 h + 0 .. 3 and
+// 16 j + 8 + 4 h + 0 .. 3, h = l / 32. One ds_read_b64_tr_b16 each: lane a of a 16-lane group g
+// addresses 4 values of d at position k0 + a / 4 and receives positions k0 .. k0 + 3 of its own d
+// (lane layout checked on the box, gemm_lds.h).
+__device__ __forceinline__ half8 frag_t(const uint4* tile, int d0, int j, int lane) {
+  using cm::gemm::lds_short4_t;
+  using cm::gemm::short4v;
+  const int a = lane % 16, h = lane / 32;
+  const int d = d0 + (lane / 16 % 2) * 16 + 4 * (a % 4);
+  const int r0 = 4 * h + a / 4, r1 = r0 + 8;  // 16 j leaves swz as it is
+  const char* t = reinterpret_cast<const char*>(tile) + j * 16 * kD * 2 + (d % 8) * 2;
+  const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_short4_t*)(t + (r0 * kCh + ((d / 8) ^ swz(r0))) * 16));
+  const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_short4_t*)(t + (r1 * kCh + ((d / 8) ^ swz(r1))) * 16));
+  const short4v v[2] = {lo, hi};
+  return __builtin_bit_cast(half8, v);
+}
+
+// Issue this thread's loads of a tile of ROWS positions from src (rows of kD fp16 in a row); NW
+// wavefronts load it together (wave = 0 .. NW - 1).
+template <int ROWS, int NW>
+__device__ __forceinline__ void load_tile(uint4* tile, const _Float16* src, int wave, int lane) {
+  constexpr int kPer = ROWS * kCh / (NW * cm::kWave);
+  static_assert(kPer * NW * cm::kWave == ROWS * kCh, "tile chunks split over the wavefronts");
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
-    const int c = (i * kNW + wave) * cm::kWave + lane;
-    const int row = c / CH, phys = c % CH;
-    const char* g = static_cast<const char*>(src) + row * row_bytes + (phys ^ swz<CH>(row)) * 16;
-    cm::gemm::dma16(g, tile + (i * kNW + wave) * cm::kWave);
+    const int c = (i * NW + wave) * cm::kWave + lane;
+    const int row = c / kCh, phys = c % kCh;
+    cm::gemm::dma16(src + row * kD + (phys ^ swz(row)) * 8, tile + (i * NW + wave) * cm::kWave);
   }
 }
 
@@ -259,13 +269,12 @@ __device__ __forceinline__ void load_vec128(uint4* slot, const void* src, int wa
 __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---------------------------------------------------------------------------------------------
-// Relayout: fp16 natural and/or transposed copies of a [heads][N][D] tensor in the padded
-// position space, and optionally Delta = rowsum(X * O) (X = dO).
+// Relayout: the fp16 copy of a [heads][N][D] tensor in the padded position space, and optionally
+// Delta = rowsum(X * O) (X = dO).
 struct Job {
   const void* src;
   int64_t sh, st;       // element strides of src (head, token); d is contiguous
-  _Float16* nat;        // [heads][n_pad][D] or null
-  _Float16* tr;         // [heads][D][n_pad] (16-groups permuted) or null
+  _Float16* nat;        // [heads][n_pad][D]
   const _Float16* o;    // with delta: O, element (t, h, d) at o[t * so_t + h * D + d]
   float* delta;         // [heads][n_pad] or null
   int64_t so_t;
@@ -282,7 +291,6 @@ struct Jobs {
 
 __global__ __launch_bounds__(256) void attn_relayout_kernel(Jobs jobs, const Rows* rows_p,
                                                             int n_tokens, int n_pad) {
-  __shared__ _Float16 tile[kD * kBlk];  // transposed staging [d][slot]
   const Rows& rows = *rows_p;
   const Where where = locate(rows, blockIdx.x, n_tokens, n_pad);
   if (!where.live) return;
@@ -358,16 +366,8 @@ __global__ __launch_bounds__(256) void attn_relayout_kernel(Jobs jobs, const Row
         x[i] = static_cast<_Float16>(ch < 8 ? rot_minus(xv[it][i], pv[i], cv[it][i], sv[it][i])
                                             : rot_plus(xv[it][i], pv[i], cv[it][i], sv[it][i]));
     }
-    if (job.nat)
-      *reinterpret_cast<half8*>(job.nat + (static_cast<int64_t>(h) * n_pad + pos0 + t) * kD +
-                                ch * 8) = x;
-    if (job.tr) {
-      // row d of the staging tile holds its 8-slot chunks XOR-swizzled by (d / 8) % 8, so the 16
-      // lanes of one token (16 values of d eight apart) write to 8 distinct banks, not one
-      const int slot = ((t & ~15) | perm16(t & 15)) ^ ((ch & 7) << 3);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) tile[(ch * 8 + i) * kBlk + slot] = x[i];
-    }
+    *reinterpret_cast<half8*>(job.nat + (static_cast<int64_t>(h) * n_pad + pos0 + t) * kD +
+                              ch * 8) = x;
     if (job.delta) {
       float d = 0.0f;
       if (ok) {
@@ -380,58 +380,69 @@ __global__ __launch_bounds__(256) void attn_relayout_kernel(Jobs jobs, const Row
       if (ch == 0) job.delta[static_cast<int64_t>(h) * n_pad + pos0 + t] = d;
     }
   }
-  if (!job.tr) return;
-  __syncthreads();
-  for (int c = threadIdx.x; c < kD * (kBlk / 8); c += 256) {
-    const int d = c / (kBlk / 8), ch = c % (kBlk / 8);
-    const int pc = ch ^ ((d >> 3) & 7);
-    *reinterpret_cast<uint4*>(job.tr + (static_cast<int64_t>(h) * kD + d) * n_pad + pos0 +
-                              ch * 8) = *reinterpret_cast<const uint4*>(tile + d * kBlk + pc * 8);
-  }
 }
 
 // ---------------------------------------------------------------------------------------------
-// The three attention kernels run four wavefronts per block in two pairs. Both pairs own the same
-// 64 queries (or keys), wavefront 2p + w the 32 of half w; the serial loop over the other side's
-// blocks is split between the pairs (pair p takes every other block), each pair double-buffers
-// its own tiles in its own LDS region, and at the end pair 1 hands its partial results to pair 0
-// through that region. Both pairs run the same number of iterations (one barrier each).
+// The attention kernels run four wavefronts per block, in the backward and in the forward's split
+// form in two pairs. Both pairs own the same 64 queries (or keys), wavefront 2p + w the 32 of half
+// w; the serial loop over the other side's blocks is split between the pairs (pair p takes every
+// other block), each pair double-buffers its own tiles in its own LDS region, and at the end pair 1
+// hands its partial results to pair 0 through the LDS. Both pairs run the same number of iterations
+// (one barrier each).
+//
+// What bounds them: below a few thousand tokens the serial chain of a block (at most one workgroup
+// per CU), above it the waits inside an iteration (fragment reads, softmax, barrier), which only the
+// SIMD's other wavefront covers: at 8191 tokens in one row, 12 heads, the backward's MFMAs take 35%
+// of the time. Backward with its relayout and head sum, one MI355X, before (one workgroup per CU,
+// transposed tiles) and now, same bits: 8191 tokens 1510 -> 995 us, 16 x 300 141 -> 108, 2048 + 1000
+// 174 -> 123, 4 rows of 154-482 51.6 -> 45.6. One pair per workgroup (four to a CU) was measured and
+// not kept: 2 x 4000 tokens 753 us against 813, but 2048 + 1000 164 against 125.
 
-// Forward. Block (b, h): 64 queries of one row, query head h (key/value head h / hpg). Pair p
-// takes the row's 64-key blocks p, p + 2, ... up to the diagonal block qb.
-constexpr int kKTile = kBlk * (kD / 8);   // K tile: 64 keys x 16 chunks
-constexpr int kVTile = kD * (kBlk / 8);   // V^T tile: 128 d x 8 chunks
+// Forward. Two forms, both with 32 queries per wavefront:
+//  - SPLIT: block (b, h) is 64 queries of one row, query head h (key/value head h / hpg); pair p
+//    takes the row's 64-key blocks p, p + 2, ... up to the diagonal block qb.
+//  - whole: 128 queries (blocks b and b + 1 of the row, b even in it), and all four wavefronts take
+//    every key block together: half the tile loads per query, no merge at the end, and half the LDS,
+//    so that a CU holds two workgroups and one's softmax runs beside the other's MFMAs.
+constexpr int kTile = kBlk * kCh;  // a tile of 64 positions
 
-__global__ __launch_bounds__(kThreads) void attn_fwd_kernel(
+template <bool SPLIT>
+__global__ __launch_bounds__(kThreads, SPLIT ? 1 : 2) void attn_fwd_kernel(
     const void* __restrict__ q, int q_dtype, int64_t sq_h, int64_t sq_t,
-    const _Float16* __restrict__ k16, const _Float16* __restrict__ vt16,
+    const _Float16* __restrict__ k16, const _Float16* __restrict__ v16,
     const Rows* __restrict__ rows_p, int n_tokens, int n_pad, int hpg, int H, float c_log2,
     _Float16* __restrict__ out, float* __restrict__ lse2, int q_padded) {
-  constexpr int kStage = kKTile + kVTile;
-  __shared__ uint4 lds[2][2][kStage];  // [pair][stage]
+  constexpr int kStage = 2 * kTile;  // K, V
+  constexpr int kSets = SPLIT ? 2 : 1;  // wavefront sets with key blocks of their own
+  constexpr int kSetWaves = 4 / kSets;
+  __shared__ uint4 lds[kSets][2][kStage];  // [set][stage]
   const Rows& rows = *rows_p;
   const int h = blockIdx.x, g = h / hpg;
   const int b = heavy_first_query_block();
   const Where where = locate(rows, b, n_tokens, n_pad);
   if (!where.live) return;
   const int qb = b - where.pstart / kBlk;
+  if (!SPLIT && qb % 2) return;  // the second half of block b - 1's queries
   const int len = where.len;
   const int p0 = where.pstart;
   const int lane = threadIdx.x % cm::kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / cm::kWave);
-  const int pair = wave >> 1, wq = wave & 1;
+  const int set = SPLIT ? wave >> 1 : 0, wq = wave % kSetWaves;
   const int hh = lane / 32, ln = lane % 32;
-  const int ql = qb * kBlk + wq * 32 + ln;  // query position in the row
+  const int q0 = qb * kBlk + wq * 32;  // the wavefront's first query in the row
+  const int ql = q0 + ln;
   const bool q_ok = ql < len;
-  const int n_it = (qb + 2) / 2;
+  // the last key block of the workgroup's queries
+  const int jb_last = SPLIT ? qb : min(qb + 1, (len - 1) / kBlk);
+  const int n_it = (jb_last + kSets) / kSets;
 
   const _Float16* kbase = k16 + (static_cast<int64_t>(g) * n_pad + p0) * kD;
-  const _Float16* vbase = vt16 + static_cast<int64_t>(g) * kD * n_pad + p0;
+  const _Float16* vbase = v16 + (static_cast<int64_t>(g) * n_pad + p0) * kD;
   auto issue = [&](int jb, int st) {
-    load_tile<kBlk, kD / 8>(lds[pair][st], kbase + jb * kBlk * kD, kD * 2, wq, lane);
-    load_tile<kD, kBlk / 8>(lds[pair][st] + kKTile, vbase + jb * kBlk, n_pad * 2, wq, lane);
+    load_tile<kBlk, kSetWaves>(lds[set][st], kbase + jb * kBlk * kD, wq, lane);
+    load_tile<kBlk, kSetWaves>(lds[set][st] + kTile, vbase + jb * kBlk * kD, wq, lane);
   };
-  if (pair <= qb) issue(pair, 0);
+  if (set <= jb_last) issue(set, 0);
 
   half8 qf[kD / 16];
   {
@@ -448,22 +459,23 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_kernel(
   float m = -__builtin_huge_valf(), l = 0.0f;  // reference max (log2 domain) and sum
 
   for (int it = 0; it < n_it; ++it) {
-    const int jb = 2 * it + pair, st = it & 1;
+    const int jb = kSets * it + set, st = it & 1;
     cm::gemm::wait_vmcnt<0>();
     cm::gemm::lds_barrier();
-    if (jb + 2 <= qb) issue(jb + 2, st ^ 1);
-    if (jb > qb) continue;  // pair 1's last iteration when qb is even
-    const uint4* kt = lds[pair][st];
-    const uint4* vt = kt + kKTile;
+    if (jb + kSets <= jb_last) issue(jb + kSets, st ^ 1);
+    // set 1's last iteration when qb is even; keys that all follow this wavefront's queries
+    if (jb > jb_last || jb * kBlk > q0 + 31) continue;
+    const uint4* kt = lds[set][st];
+    const uint4* vt = kt + kTile;
     floatx16 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       s[t] = zero16();
 #pragma unroll
       for (int ds = 0; ds < kD / 16; ++ds)
-        s[t] = mfma(frag<kD / 8>(kt, t * 32 + ln, ds * 2 + hh), qf[ds], s[t]);
+        s[t] = mfma(frag(kt, t * 32 + ln, ds * 2 + hh), qf[ds], s[t]);
     }
-    if (jb == qb) {  // the diagonal block: keys after the query are masked
+    if (jb * kBlk + kBlk - 1 > q0) {  // a diagonal block: keys after the query are masked
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -511,24 +523,31 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_kernel(
     for (int dt = 0; dt < kD / 32; ++dt)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
-        o[dt] = mfma(frag<kBlk / 8>(vt, dt * 32 + ln, ks * 2 + hh), pf[ks], o[dt]);
+        o[dt] = mfma(frag_t(vt, dt * 32, ks, lane), pf[ks], o[dt]);
   }
 
-  // pair 1 hands (o, m, l) of its blocks to pair 0 through its LDS region
-  cm::gemm::lds_barrier();
-  float* xf = reinterpret_cast<float*>(lds[1][0]) + wq * 66 * cm::kWave + lane;
-  if (pair == 1) {
+  float* xf = nullptr;
+  float mt = m, a0 = 1.0f, a1 = 0.0f;
+  if constexpr (SPLIT) {
+    // set 1 hands (o, m, l) of its blocks to set 0 through its LDS region
+    cm::gemm::lds_barrier();
+    xf = reinterpret_cast<float*>(lds[kSets - 1][0]) + wq * 66 * cm::kWave + lane;
+    if (set == 1) {
 #pragma unroll
-    for (int i = 0; i < kD / 2; ++i) xf[i * cm::kWave] = o[i / 16][i % 16];
-    xf[64 * cm::kWave] = m;
-    xf[65 * cm::kWave] = l;
+      for (int i = 0; i < kD / 2; ++i) xf[i * cm::kWave] = o[i / 16][i % 16];
+      xf[64 * cm::kWave] = m;
+      xf[65 * cm::kWave] = l;
+    }
+    cm::gemm::lds_barrier();
+    if (set == 1) return;
+    const float m1 = xf[64 * cm::kWave], l1 = xf[65 * cm::kWave];
+    mt = fmaxf(m, m1);
+    a0 = exp2_raw(m - mt);
+    a1 = exp2_raw(m1 - mt);  // 0 when set 1 had none
+    l = l * a0 + l1 * a1;
   }
-  cm::gemm::lds_barrier();
-  if (pair == 1) return;
-  const float m1 = xf[64 * cm::kWave], l1 = xf[65 * cm::kWave];
-  const float mt = fmaxf(m, m1);
-  const float a0 = exp2_raw(m - mt), a1 = exp2_raw(m1 - mt);  // a1 = 0 when pair 1 had none
-  l = l * a0 + l1 * a1;
+  // positions past the row's padded blocks are another row's
+  if (!SPLIT && q0 >= (len + kBlk - 1) / kBlk * kBlk) return;
   if (hh == 0) lse2[static_cast<int64_t>(h) * n_pad + p0 + ql] = mt + __log2f(l);
   if (!q_ok) return;
   const float inv = 1.0f / l;
@@ -542,7 +561,9 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int e = g4 * 4 + i;
-        v[i] = static_cast<_Float16>((o[dt][e] * a0 + xf[(dt * 16 + e) * cm::kWave] * a1) * inv);
+        float ov = o[dt][e];
+        if constexpr (SPLIT) ov = ov * a0 + xf[(dt * 16 + e) * cm::kWave] * a1;
+        v[i] = static_cast<_Float16>(ov * inv);
       }
       *reinterpret_cast<h4*>(orow + dt * 32 + g4 * 8 + hh * 4) = v;
     }
@@ -553,20 +574,16 @@ __global__ __launch_bounds__(kThreads) void attn_fwd_kernel(
 // row's 32-query tiles qt_first + p, qt_first + p + 2, ... from the block's first key on. Writes
 // the head's partial dK (times the softmax scale) and dV, fp32 [H][n_pad][D]. Queries past the
 // row end need no mask: their q and dO rows are zero, so they add exactly zero.
-constexpr int kQTile = 32 * (kD / 8);   // Q / dO tile: 32 queries x 16 chunks
-constexpr int kQTTile = kD * (32 / 8);  // Q^T / dO^T tile: 128 d x 4 chunks
-constexpr int kDkdvVec = 2 * kQTile + 2 * kQTTile;  // lse (8 chunks) and Delta (8) follow
+constexpr int kHalf = 32 * kCh;      // a tile of 32 positions
+constexpr int kDkdvVec = 2 * kHalf;  // Q and dO; lse (8 chunks) and Delta (8) follow
 constexpr int kDkdvStage = kDkdvVec + 16;
 
 // The operands of the backward's dK/dV and dQ blocks (one launch runs both).
 struct BwdArgs {
   const _Float16* q16;
-  const _Float16* qt16;
   const _Float16* do16;
-  const _Float16* dot16;
   const _Float16* k16;
   const _Float16* v16;
-  const _Float16* kt16;
   const float* lse2;
   const float* delta;
   const Rows* rows;
@@ -579,15 +596,13 @@ struct BwdArgs {
   float* dq_rot;    // fused RoPE: dQ of the rotated q, [H][n_pad][D] fp32, or null
 };
 
-// raw: the workgroup's LDS, 4 stages of kDkdvStage
+// raw: the workgroup's LDS, 2 stages of kDkdvStage per pair
 __device__ __forceinline__ void bwd_dkdv_block(const BwdArgs& a, int h, int b, uint4* raw) {
   constexpr int kVec = kDkdvVec;
   constexpr int kStage = kDkdvStage;
   auto lds = reinterpret_cast<uint4 (*)[2][kStage]>(raw);  // [pair][stage]
   const _Float16* __restrict__ q16 = a.q16;
-  const _Float16* __restrict__ qt16 = a.qt16;
   const _Float16* __restrict__ do16 = a.do16;
-  const _Float16* __restrict__ dot16 = a.dot16;
   const _Float16* __restrict__ k16 = a.k16;
   const _Float16* __restrict__ v16 = a.v16;
   const float* __restrict__ lse2 = a.lse2;
@@ -612,13 +627,8 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdArgs& a, int h, int b, u
   auto issue = [&](int qt, int st) {
     const int64_t pos = p0 + qt * 32;
     uint4* t = lds[pair][st];
-    load_tile<32, kD / 8>(t, q16 + (hq + pos) * kD, kD * 2, wq, lane);
-    load_tile<32, kD / 8>(t + kQTile, do16 + (hq + pos) * kD, kD * 2, wq, lane);
-    load_tile<kD, 32 / 8>(t + 2 * kQTile, qt16 + static_cast<int64_t>(h) * kD * n_pad + pos,
-                          n_pad * 2, wq, lane);
-    load_tile<kD, 32 / 8>(t + 2 * kQTile + kQTTile,
-                          dot16 + static_cast<int64_t>(h) * kD * n_pad + pos, n_pad * 2, wq,
-                          lane);
+    load_tile<32, 2>(t, q16 + (hq + pos) * kD, wq, lane);
+    load_tile<32, 2>(t + kHalf, do16 + (hq + pos) * kD, wq, lane);
     load_vec128(t + kVec, lse2 + hq + pos, wq, lane);
     load_vec128(t + kVec + 8, delta + hq + pos, wq, lane);
   };
@@ -651,17 +661,15 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdArgs& a, int h, int b, u
     if (qt >= qt_end) continue;           // pair 1's last iteration
     if (qt * 32 + 31 < key0) continue;    // the tile's queries all precede this wavefront's keys
     const uint4* qs = lds[pair][st];
-    const uint4* dos = qs + kQTile;
-    const uint4* qts = qs + 2 * kQTile;
-    const uint4* dots = qts + kQTTile;
+    const uint4* dos = qs + kHalf;
     // lse and Delta of the lane's 16 queries qt*32 + (e/4)*8 + hh*4 + e%4
     const float4* lv = reinterpret_cast<const float4*>(qs + kVec);
     const float4* dlv = reinterpret_cast<const float4*>(qs + kVec + 8);
     floatx16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int ds = 0; ds < kD / 16; ++ds) {
-      s = mfma(frag<kD / 8>(qs, ln, ds * 2 + hh), kf[ds], s);
-      dp = mfma(frag<kD / 8>(dos, ln, ds * 2 + hh), vf[ds], dp);
+      s = mfma(frag(qs, ln, ds * 2 + hh), kf[ds], s);
+      dp = mfma(frag(dos, ln, ds * 2 + hh), vf[ds], dp);
     }
     const bool diag = qt * 32 < key0 + 31;  // some query of the tile precedes some key
 #pragma unroll
@@ -687,13 +695,15 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdArgs& a, int h, int b, u
     for (int dt = 0; dt < kD / 32; ++dt)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        dv[dt] = mfma(frag<32 / 8>(dots, dt * 32 + ln, j * 2 + hh), pf[j], dv[dt]);
-        dk[dt] = mfma(frag<32 / 8>(qts, dt * 32 + ln, j * 2 + hh), sf[j], dk[dt]);
+        dv[dt] = mfma(frag_t(dos, dt * 32, j, lane), pf[j], dv[dt]);
+        dk[dt] = mfma(frag_t(qs, dt * 32, j, lane), sf[j], dk[dt]);
       }
   }
 
+  // both wavefronts of pair 1 hand over 128 values per lane: 64 KiB, over both pairs' tiles
+  static_assert(2 * 128 * cm::kWave * sizeof(float) <= sizeof(uint4) * 4 * kStage, "fits");
   cm::gemm::lds_barrier();
-  float* xf = reinterpret_cast<float*>(lds[1][0]) + wq * 128 * cm::kWave + lane;
+  float* xf = reinterpret_cast<float*>(raw) + wq * 128 * cm::kWave + lane;
   if (pair == 1) {
 #pragma unroll
     for (int i = 0; i < kD / 2; ++i) {
@@ -727,10 +737,7 @@ __device__ __forceinline__ void bwd_dkdv_block(const BwdArgs& a, int h, int b, u
 // ---------------------------------------------------------------------------------------------
 // Backward, dQ. Block (b, h): 64 queries of one row, head h; pair p takes the 32-key tiles p,
 // p + 2, ... up to the diagonal.
-constexpr int kKVTile = 32 * (kD / 8);  // K / V tile: 32 keys x 16 chunks
-constexpr int kKTTile = kD * (32 / 8);  // K^T tile: 128 d x 4 chunks
-
-constexpr int kDqStage = 2 * kKVTile + kKTTile;
+constexpr int kDqStage = 2 * kHalf;  // K, V
 
 template <typename OT>
 __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uint4* raw) {
@@ -740,7 +747,6 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
   const _Float16* __restrict__ do16 = a.do16;
   const _Float16* __restrict__ k16 = a.k16;
   const _Float16* __restrict__ v16 = a.v16;
-  const _Float16* __restrict__ kt16 = a.kt16;
   const float* __restrict__ lse2 = a.lse2;
   const float* __restrict__ delta = a.delta;
   const int n_tokens = a.n_tokens, n_pad = a.n_pad, tok_major = a.tok_major;
@@ -765,10 +771,8 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
   auto issue = [&](int kt, int st) {
     const int64_t pos = p0 + kt * 32;
     uint4* t = lds[pair][st];
-    load_tile<32, kD / 8>(t, k16 + (gk + pos) * kD, kD * 2, wq, lane);
-    load_tile<32, kD / 8>(t + kKVTile, v16 + (gk + pos) * kD, kD * 2, wq, lane);
-    load_tile<kD, 32 / 8>(t + 2 * kKVTile, kt16 + static_cast<int64_t>(g) * kD * n_pad + pos,
-                          n_pad * 2, wq, lane);
+    load_tile<32, 2>(t, k16 + (gk + pos) * kD, wq, lane);
+    load_tile<32, 2>(t + kHalf, v16 + (gk + pos) * kD, wq, lane);
   };
   const int n_it = qb + 1;  // 32-key tiles 0 .. 2 qb + 1, every other one per pair
   issue(pair, 0);
@@ -792,13 +796,12 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
     if (kt + 2 < 2 * n_it) issue(kt + 2, st ^ 1);
     if (kt * 32 > q0 + 31) continue;  // the tile's keys all follow this wavefront's queries
     const uint4* ks = lds[pair][st];
-    const uint4* vs = ks + kKVTile;
-    const uint4* kts = ks + 2 * kKVTile;
+    const uint4* vs = ks + kHalf;
     floatx16 s = zero16(), dp = zero16();
 #pragma unroll
     for (int ds = 0; ds < kD / 16; ++ds) {
-      s = mfma(frag<kD / 8>(ks, ln, ds * 2 + hh), qf[ds], s);
-      dp = mfma(frag<kD / 8>(vs, ln, ds * 2 + hh), of[ds], dp);
+      s = mfma(frag(ks, ln, ds * 2 + hh), qf[ds], s);
+      dp = mfma(frag(vs, ln, ds * 2 + hh), of[ds], dp);
     }
     const bool diag = kt * 32 + 31 > q0;  // some key of the tile follows some query
 #pragma unroll
@@ -814,10 +817,11 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
     for (int dt = 0; dt < kD / 32; ++dt)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        acc[dt] = mfma(frag<32 / 8>(kts, dt * 32 + ln, j * 2 + hh), sf[j], acc[dt]);
+        acc[dt] = mfma(frag_t(ks, dt * 32, j, lane), sf[j], acc[dt]);
   }
 
   cm::gemm::lds_barrier();
+  static_assert(2 * 64 * cm::kWave * sizeof(float) <= sizeof(uint4) * 2 * kStage, "fits");
   float* xf = reinterpret_cast<float*>(lds[1][0]) + wq * 64 * cm::kWave + lane;
   if (pair == 1) {
 #pragma unroll
@@ -859,8 +863,10 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
 // CUs the other's heavy blocks leave idle. The LDS holds the larger of the two stage rings.
 constexpr int kBwdLds = 4 * (kDkdvStage > kDqStage ? kDkdvStage : kDqStage);
 
+// The LDS holds both pairs' double buffers (65 KiB: two workgroups per CU, so that one's softmax
+// and LDS waits run beside the other's MFMAs).
 template <typename OT>
-__global__ __launch_bounds__(kThreads) void attn_bwd_kernel(BwdArgs a) {
+__global__ __launch_bounds__(kThreads, 2) void attn_bwd_kernel(BwdArgs a) {
   __shared__ uint4 raw[kBwdLds];
   const int x = blockIdx.x;
   if (x < a.H) {
@@ -980,13 +986,22 @@ struct Workspace {
   }
 };
 
-// k16 and vt16, and q16 (the rotated q of a fused RoPE)
+// The forward's form, by the launch's 64-query blocks times heads (the rows' lengths are only on the
+// device). The split form has one workgroup per block and the shorter serial chain, the whole form
+// half as many workgroups, two to a CU. Split / whole, forward with its relayout, us: 252 (4 rows of
+// 154-482 tokens, 12 heads) 19.8 / 22.1; 588 (2048 + 1000) 52 / 58; 672 (1500, 28 heads) 53 / 50;
+// 768 (8 x 512) 43 / 36; 960 (16 x 300) 44 / 36; 1316 (3000, 28 heads) 146 / 118; 1536 (8191) 355 /
+// 345. The one loss above the line is 1008 (2 x 2000, 16 heads): 84 / 86.
+constexpr int64_t kSplitBelow = 768;
+
+// k16 and v16, and q16 (the rotated q of a fused RoPE)
 size_t fwd_ws_bytes(int64_t n_pad, int H, int G) {
   return 2 * align256(static_cast<size_t>(G) * n_pad * kD * 2) +
          align256(static_cast<size_t>(H) * n_pad * kD * 2);
 }
 
-// q16, do16, qt16, dot16; k16, v16, kt16; Delta; dK / dV partials and the fused RoPE's dQ
+// q16, do16; k16, v16; Delta; dK / dV partials and the fused RoPE's dQ. The size is the interface's:
+// it also covers two query and one key array that no kernel uses any more.
 size_t bwd_ws_bytes(int64_t n_pad, int H, int G) {
   const size_t hq = align256(static_cast<size_t>(H) * n_pad * kD * 2);
   const size_t gk = align256(static_cast<size_t>(G) * n_pad * kD * 2);
@@ -1057,16 +1072,16 @@ int fwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
   hipStream_t s = static_cast<hipStream_t>(stream);
   Workspace ws{static_cast<char*>(workspace), 0, static_cast<size_t>(workspace_bytes)};
   _Float16* k16 = ws.take<_Float16>(static_cast<size_t>(G) * n_pad * kD);
-  _Float16* vt16 = ws.take<_Float16>(static_cast<size_t>(G) * n_pad * kD);
+  _Float16* v16 = ws.take<_Float16>(static_cast<size_t>(G) * n_pad * kD);
   _Float16* q16 = ws.take<_Float16>(static_cast<size_t>(H) * n_pad * kD);
   const Rope none{nullptr, nullptr, 0};
   const bool fused = rope.cos != nullptr;
   // with a fused RoPE, q and k are rotated on their way into the fp16 copies, and the query
   // kernel reads q's copy (in the padded positions) in place of q
   Jobs jobs{};
-  jobs.job[0] = Job{k, sk_h, sk_t, k16, nullptr, nullptr, nullptr, 0, k_dtype, G, rope};
-  jobs.job[1] = Job{v, sv_h, sv_t, nullptr, vt16, nullptr, nullptr, 0, v_dtype, G, none};
-  jobs.job[2] = Job{q, sq_h, sq_t, q16, nullptr, nullptr, nullptr, 0, q_dtype, H, rope};
+  jobs.job[0] = Job{k, sk_h, sk_t, k16, nullptr, nullptr, 0, k_dtype, G, rope};
+  jobs.job[1] = Job{v, sv_h, sv_t, v16, nullptr, nullptr, 0, v_dtype, G, none};
+  jobs.job[2] = Job{q, sq_h, sq_t, q16, nullptr, nullptr, 0, q_dtype, H, rope};
   jobs.first[1] = G;
   jobs.first[2] = 2 * G;
   jobs.n = fused ? 3 : 2;
@@ -1077,9 +1092,10 @@ int fwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
                      s, jobs, rows, nt, np);
   if (int st = cm::launch_status()) return st;
   const void* qa = fused ? static_cast<const void*>(q16) : q;
-  hipLaunchKernelGGL(attn_fwd_kernel, dim3(H, n_blocks), dim3(kThreads), 0, s, qa,
+  const auto kernel = static_cast<int64_t>(H) * n_blocks < kSplitBelow ? attn_fwd_kernel<true> : attn_fwd_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(H, n_blocks), dim3(kThreads), 0, s, qa,
                      fused ? CM_F16 : q_dtype, fused ? static_cast<int64_t>(n_pad) * kD : sq_h,
-                     fused ? static_cast<int64_t>(kD) : sq_t, k16, vt16, rows, nt, np, H / G, H,
+                     fused ? static_cast<int64_t>(kD) : sq_t, k16, v16, rows, nt, np, H / G, H,
                      scale * 1.4426950408889634f, static_cast<_Float16*>(out), lse2,
                      fused ? 1 : 0);
   return cm::launch_status();
@@ -1141,11 +1157,8 @@ int bwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
   const size_t nq = static_cast<size_t>(H) * n_pad * kD, nk = static_cast<size_t>(G) * n_pad * kD;
   _Float16* q16 = ws.take<_Float16>(nq);
   _Float16* do16 = ws.take<_Float16>(nq);
-  _Float16* qt16 = ws.take<_Float16>(nq);
-  _Float16* dot16 = ws.take<_Float16>(nq);
   _Float16* k16 = ws.take<_Float16>(nk);
   _Float16* v16 = ws.take<_Float16>(nk);
-  _Float16* kt16 = ws.take<_Float16>(nk);
   float* delta = ws.take<float>(static_cast<size_t>(H) * n_pad);
   float* dk_part = ws.take<float>(nq);
   float* dv_part = ws.take<float>(nq);
@@ -1159,12 +1172,12 @@ int bwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
   // dO and O: [N][H][D] contiguous (the forward's output layout); q and k rotated again on the
   // way when the RoPE is fused
   Jobs jobs{};
-  jobs.job[0] = Job{q, sq_h, sq_t, q16, qt16, nullptr, nullptr, 0, q_dtype, H, rope};
-  jobs.job[1] = Job{dout, kD, static_cast<int64_t>(H) * kD, do16, dot16,
+  jobs.job[0] = Job{q, sq_h, sq_t, q16, nullptr, nullptr, 0, q_dtype, H, rope};
+  jobs.job[1] = Job{dout, kD, static_cast<int64_t>(H) * kD, do16,
                     static_cast<const _Float16*>(out), delta, static_cast<int64_t>(H) * kD,
                     CM_F16, H, none};
-  jobs.job[2] = Job{k, sk_h, sk_t, k16, kt16, nullptr, nullptr, 0, k_dtype, G, rope};
-  jobs.job[3] = Job{v, sv_h, sv_t, v16, nullptr, nullptr, nullptr, 0, v_dtype, G, none};
+  jobs.job[2] = Job{k, sk_h, sk_t, k16, nullptr, nullptr, 0, k_dtype, G, rope};
+  jobs.job[3] = Job{v, sv_h, sv_t, v16, nullptr, nullptr, 0, v_dtype, G, none};
   jobs.first[1] = H;
   jobs.first[2] = 2 * H;
   jobs.first[3] = 2 * H + G;
@@ -1173,7 +1186,7 @@ int bwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
                      rows, nt, np);
   if (int st = cm::launch_status()) return st;
   const int tm = grads_token_major ? 1 : 0;
-  const BwdArgs ba{q16,  qt16, do16, dot16, k16, v16, kt16, lse2, delta, rows, nt, np, H / G, H,
+  const BwdArgs ba{q16, do16, k16, v16, lse2, delta, rows, nt, np, H / G, H,
                    scale * 1.4426950408889634f, scale, dk_part, dv_part, dq, tm, dq_rot};
   if (dq_dtype == CM_F32) {
     hipLaunchKernelGGL(attn_bwd_kernel<float>, dim3(2 * H, n_blocks), dim3(kThreads), 0, s, ba);

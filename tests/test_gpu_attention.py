@@ -347,3 +347,30 @@ def test_fused_rope_equals_rope_then_attention(dev, lengths, layout):
     for a, b, name in ((q1, q2, "dq"), (k1, k2, "dk"), (v1, v2, "dv")):
         assert a.grad.dtype == b.grad.dtype, name
         assert torch.equal(a.grad, b.grad), (name, float((a.grad.float() - b.grad.float()).abs().max()))
+
+
+# 64-query blocks times heads on both sides of the line (768) where the forward takes 128 queries per
+# workgroup; rows of an odd number of blocks, of one token, and just over and under whole blocks
+WHOLE_BLOCKS = [
+    ([512] * 7 + [448], 12),  # 63 x 12
+    ([512] * 8, 12),  # 64 x 12
+    ([1, 64, 65, 127, 128, 129, 192, 193, 3300, 1], 12),
+    ([2049], 28),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths,heads", WHOLE_BLOCKS, ids=lambda x: str(x)[:24])
+def test_forward_forms_match_fp32(dev, lengths, heads):
+    from claudemaxing_amd.attention import packed_causal_attention
+
+    q, k, v, do = _inputs(dev, sum(lengths), 5, heads=heads, groups=heads // (6 if heads == 12 else 7))
+    out = packed_causal_attention(q, k, v, _bounds(lengths))
+    out.backward(do)
+    ref, grads = _reference(q, k, v, lengths, do, 128 ** -0.5)
+    # the probabilities and the result are rounded to fp16 (2^-11 each, of values up to max |v|)
+    bound = 2 ** -10 * float(v.detach().float().abs().max())
+    assert _err(out, ref) <= bound
+    # the gradients' roundings are of the same kind (P, dS, the result): 5e-4 of the norm measured
+    for got, want in zip((q.grad, k.grad, v.grad), grads):
+        assert float((got.float() - want).norm() / want.norm()) <= 2e-3

@@ -13,7 +13,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libclaudemaxing_amd.so"
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 F32, F16, BF16, U8, I32, I64 = 0, 1, 2, 3, 4, 5
 _DTYPE_CODES = {
@@ -51,6 +51,7 @@ class NF4Weight(ctypes.Structure):
 _PW = ctypes.POINTER(NF4Weight)
 _PP = ctypes.POINTER(ctypes.c_void_p)
 _PL = ctypes.POINTER(ctypes.c_int64)
+_PI = ctypes.POINTER(ctypes.c_int)
 
 # name -> (restype, argtypes); mirrors include/claudemaxing_amd.h
 SIGNATURES = {
@@ -104,6 +105,7 @@ SIGNATURES = {
                                      _PP, _P, _P]),
     "cm_lora_fused_bwd1_multi": (_I, [_L, _I, _F, _I, _PP, _PP, _PP, _PP, _PP, _P, _P]),
     "cm_lora_fused_bwd2": (_I, [_P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _F, _P]),
+    "cm_lora_fused_bwd2_multi": (_I, [_P, _P, _P, _L, _I, _I, _F, _I, _PP, _PP, _PP, _PP, _P]),
     "cm_attn_workspace_bytes": (_L, [_L, _I, _I, _I, _I]),
     "cm_nf4_linear_fwd": (_I, [_P, _L, _L, _PW, _I, _PP, _PP, _PL, _I, _P, _L, _P]),
     "cm_nf4_linear_bwd": (_I, [_PP, _PL, _L, _PW, _I, _P, _L, _I, _P, _L, _P]),
@@ -112,8 +114,11 @@ SIGNATURES = {
     "cm_probe_mfma_f16": (_I, [_P, _I, _I, _P, _P]),
     "cm_probe_mfma_f16_flops": (_L, [_I, _I]),
     "cm_probe_launch": (_I, [_I, _I, _P]),
+    "cm_linear_f16_fwd": (_I, [_P, _L, _L, _I, _P, _I, _PI, _PP, _PP, _PL, _P]),
+    "cm_linear_f16_bwd": (_I, [_PP, _PL, _L, _I, _PI, _P, _I, _P, _L, _P]),
     "cm_nf4_scale_map": (_I, [_PW, _P, _P]),
     "cm_nf4_dequant_group": (_I, [_PW, _I, _PP, _I, _P]),
+    "cm_nf4_expand_rows": (_I, [_PW, _I, _P, _I, _P]),
 }
 
 _lock = threading.Lock()

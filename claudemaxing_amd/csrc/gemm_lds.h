@@ -156,12 +156,48 @@ struct DmaTile {
   }
 };
 
+// Direct loads of a row-major LDS tile from a SegRows operand: as DmaTile, but a lane keeps its
+// (clamped) rows, because the row stride changes with the stage's segment: one multiply-add per
+// instruction.
+template <int ROWS, int NW, int BK>
+struct DmaTileSeg {
+  using L = LdsTile<BK, false, ROWS>;
+  static constexpr int kPer = ROWS * L::kRC / (NW * kWave);
+  static constexpr int kRowStep = NW * kWave / L::kRC;
+  static_assert(kPer * NW * kWave == ROWS * L::kRC, "tile chunks must split over the wavefronts");
+  static_assert(NW >= 2, "one swizzled column per lane needs a row step of 16 or more");
+  int row[kPer];
+  int col0;
+
+  template <class Src>
+  __device__ __forceinline__ void init(const Src& src, int r0, int wave, int lane) {
+    const int c = wave * kWave + lane, row0 = c / L::kRC;
+    col0 = ((c % L::kRC) ^ L::swz(row0)) * 8;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) row[i] = min(row0 + i * kRowStep, src.rows - 1 - r0);
+  }
+  template <class Src>
+  __device__ __forceinline__ void issue_inside(const Src& src, int r0, int k0, uint4* tile,
+                                               int wave, int i) const {
+    int64_t ld;
+    const _Float16* base = src.at(r0, k0, ld);
+    const uint32_t off = (row[i] * static_cast<uint32_t>(ld) + col0) * 2;
+    dma16(reinterpret_cast<const char*>(base) + off, tile + (i * NW + wave) * kWave);
+  }
+  template <class Src>
+  __device__ __forceinline__ void issue(const Src& src, int r0, int k0, uint4* tile, int wave,
+                                        int i, bool) const {
+    issue_inside(src, r0, k0, tile, wave, i);  // segments are whole stages
+  }
+};
+
 // Direct loads of a k-major operand (KMajor): the LDS tile is BK rows (k) of BN fp16 (n), row by
-// row, with the 32-byte segments of a row XOR-swizzled by kswz(k) = 2 ((k >> 1) & 1) within
-// aligned groups of four segments. A transposing fragment read (frag_kmajor) has its 16-lane
-// groups read rows k .. k + 3 (k a multiple of 4) at one 32-byte segment and the next, so with
-// this swizzle the 8 (row, segment) pieces a 32-lane half serves at once cover the 64 banks
-// exactly once. Instruction i of a lane fills slot c = (i NW + wave) 64 + lane of the tile: row
+// row, with the 32-byte segments of a row XOR-swizzled by kswz(k): 2 (k & 3) where rows are whole
+// multiples of 256 bytes (the 64 banks), else 2 ((k >> 1) & 1) (neighbouring rows of an odd number
+// of 128-byte halves already start half the banks apart). A transposing fragment read
+// (frag_kmajor) has its 16-lane groups read rows k .. k + 3 (k a multiple of 4) at one 32-byte
+// segment and the next, so with this swizzle the 8 (row, segment) pieces a 32-lane half serves at
+// once cover the 64 banks exactly once. Instruction i of a lane fills slot c = (i NW + wave) 64 + lane of the tile: row
 // c / (BN / 8), physical slot c % (BN / 8). As in DmaTile, a lane keeps one byte offset per
 // instruction; chunks past the operand's last n are read from its last whole chunk.
 template <int BN, int NW, int BK>
@@ -171,7 +207,9 @@ struct DmaTileK {
   static constexpr int kPer = kChunks / (NW * kWave);
   static_assert(kPer * NW * kWave == kChunks, "tile chunks must split over the wavefronts");
   static_assert(BN % 64 == 0, "rows of whole groups of four 32-byte segments");
-  static __device__ __forceinline__ int kswz(int k) { return ((k >> 1) & 1) * 2; }
+  static __device__ __forceinline__ int kswz(int k) {
+    return BN % 128 == 0 ? (k & 3) * 2 : ((k >> 1) & 1) * 2;
+  }
   uint32_t off[kPer];  // byte offset of the lane's chunk of instruction i from the stage origin
   int krow[kPer];
 
@@ -308,8 +346,10 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   constexpr int KS = BK / 16;  // MFMA substeps per stage
   static_assert(TM * 32 == WTM && TN * 32 == WTN, "wave tiles are multiples of 32");
   static_assert(SB >= 2 && (SA == SB || SA == SB + 1), "A's ring is B's or one stage deeper");
+  static_assert(NW * kWave >= 128, "tiles are loaded by at least two wavefronts");
   constexpr int kTileA = BM * LA::kRC, kTileB = BN * LB::kRC;  // uint4 per stage
-  using TA = DmaTile<BM, NW, BK, SrcA::kChunkMajor>;
+  using TA = std::conditional_t<SrcA::kSegmented, DmaTileSeg<BM, NW, BK>,
+                                DmaTile<BM, NW, BK, SrcA::kChunkMajor>>;
   static_assert(!SrcA::kKMajor, "a k-major operand is B");
   using TB = std::conditional_t<SrcB::kKMajor, DmaTileK<BN, NW, BK>,
                                 DmaTile<BN, NW, BK, SrcB::kChunkMajor>>;
@@ -317,8 +357,9 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   constexpr int kDmaB = TB::kPer;
   constexpr int kDma = kDmaA + kDmaB;
   constexpr int DA = SA - 1, DB = SB - 1;  // stages from issue to use
-  // loads of stage kt + 1 that may still be in flight when stage kt is needed
-  constexpr int kLate = DA > DB ? kDmaA : 0;
+  // loads of later stages that may still be in flight when stage kt is needed: those issued after
+  // B's of stage kt
+  constexpr int kLate = (DB - 1) * kDma + (DA > DB ? kDmaA : 0);
   constexpr int NM = TM * TN, NR = TM + TN;  // MFMAs and fragments per substep
   constexpr int kSlots = NM > NR ? NM : NR;
   const int m0 = tm * BM, n0 = tn * BN;
@@ -344,19 +385,23 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   // monotonic in the stage, so the last stage decides); the main loop then issues its loads with
   // no bounds selection.
   const bool all_inside = n_kt > 0 && inside_a(n_kt - 1) && inside_b(n_kt - 1);
-  auto load_a = [&](int kt, int i, auto edge) {
+  // load instruction i of an operand's stage kt into ring slot `slot`
+  auto load_a = [&](int kt, int slot, int i, auto edge) {
     const int k0 = k_begin + kt * BK;
-    if (i >= TA::kPer) fx.issue(k0, kt % SA);
+    if (i >= TA::kPer) fx.issue(k0, slot);
     else if constexpr (decltype(edge)::value)
-      la.issue(A, m0, k0, lds + (kt % SA) * kTileA, wave, i, inside_a(kt));
-    else la.issue_inside(A, m0, k0, lds + (kt % SA) * kTileA, wave, i);
+      la.issue(A, m0, k0, lds + slot * kTileA, wave, i, inside_a(kt));
+    else la.issue_inside(A, m0, k0, lds + slot * kTileA, wave, i);
   };
-  auto load_b = [&](int kt, int i, auto edge) {
+  auto load_b = [&](int kt, int slot, int i, auto edge) {
     const int k0 = k_begin + kt * BK;
     if constexpr (decltype(edge)::value)
-      lb.issue(B, n0, k0, lds_b + (kt % SB) * kTileB, wave, i, inside_b(kt));
-    else lb.issue_inside(B, n0, k0, lds_b + (kt % SB) * kTileB, wave, i);
+      lb.issue(B, n0, k0, lds_b + slot * kTileB, wave, i, inside_b(kt));
+    else lb.issue_inside(B, n0, k0, lds_b + slot * kTileB, wave, i);
   };
+  // ring slots of the current stage (counted up: a remainder by three per use costs more); the
+  // stage loaded SA - 1 ahead goes into the slot before it
+  int slot_a = 0, slot_b = 0;
   const int arow = wm * WTM + lane % 32, brow = wn * WTN + lane % 32;
   half8 af[2][TM], bf[2][TN];
   // fragment r of substep ks, alternately of A and of B while both have one left: is_a(r) / its
@@ -364,13 +409,13 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   constexpr int kBoth = TM < TN ? TM : TN;
   auto is_a = [](int r) { return r < 2 * kBoth ? r % 2 == 0 : TM > TN; };
   auto index_of = [](int r) { return r < 2 * kBoth ? r / 2 : r - kBoth; };
-  auto read = [&](int kt, int ks, int buf, auto rc) {
+  auto read = [&](int ks, int buf, auto rc) {
     constexpr int r = decltype(rc)::value;
     const int ch = ks * 2 + lane / 32, x = index_of(r);
     if (is_a(r)) {
-      af[buf][x] = LA::frag(lds + (kt % SA) * kTileA, arow + x * 32, ch);
+      af[buf][x] = LA::frag(lds + slot_a * kTileA, arow + x * 32, ch);
     } else {
-      const uint4* Bs = lds_b + (kt % SB) * kTileB;
+      const uint4* Bs = lds_b + slot_b * kTileB;
       if constexpr (SrcB::kKMajor) bf[buf][x] = frag_kmajor<BN>(Bs, wn * WTN + x * 32, ks, lane);
       else bf[buf][x] = LB::frag(Bs, brow + x * 32, ch);
     }
@@ -385,11 +430,11 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
     constexpr int s = decltype(sc)::value;
     if (s < DB && s < n_kt) {
 #pragma unroll
-      for (int i = 0; i < kDmaB; ++i) load_b(s, i, std::true_type{});
+      for (int i = 0; i < kDmaB; ++i) load_b(s, s, i, std::true_type{});
     }
     if (s < n_kt) {
 #pragma unroll
-      for (int i = 0; i < kDmaA; ++i) load_a(s, i, std::true_type{});
+      for (int i = 0; i < kDmaA; ++i) load_a(s, s, i, std::true_type{});
     }
   });
 
@@ -400,20 +445,22 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   // both, 1 B's alone, 0 none.
   auto load = [&](int kt, int q, auto loads, auto edge) {
     if (q < kDmaB) {
-      if constexpr (decltype(loads)::value >= 1) load_b(kt + DB, q, edge);
+      if constexpr (decltype(loads)::value >= 1)
+        load_b(kt + DB, slot_b == 0 ? SB - 1 : slot_b - 1, q, edge);
     } else {
-      if constexpr (decltype(loads)::value == 2) load_a(kt + DA, q - kDmaB, edge);
+      if constexpr (decltype(loads)::value == 2)
+        load_a(kt + DA, slot_a == 0 ? SA - 1 : slot_a - 1, q - kDmaB, edge);
     }
   };
-  constexpr int kSpread = KS * NM / (DA > DB ? 1 : 2);  // MFMA slots the loads are spread over
+  constexpr int kSpread = KS * NM / (DA > 1 ? 1 : 2);  // MFMA slots the loads are spread over
   // Group g of stage kt: reads the fragments of substep g (an FX is applied a few slots after its
   // fragment's read), multiplies those of the substep before.
   auto group = [&](int kt, auto gc, auto multiply, auto loads, auto edge) {
     constexpr int g = decltype(gc)::value, buf = g & 1;
-    if constexpr (g == 0) fx.fetch(kt % SA);
+    if constexpr (g == 0) fx.fetch(slot_a);
     static_for<kSlots>([&](auto mc) {
       constexpr int m = decltype(mc)::value;
-      if constexpr (m < NR) read(kt, g, buf, mc);
+      if constexpr (m < NR) read(g, buf, mc);
       if constexpr (m < NM && decltype(multiply)::value) mfma(buf ^ 1, m);
       if constexpr (FX::kDma > 0) {
         constexpr int kLag = kSlots - NR < 5 ? kSlots - NR : 5;
@@ -430,7 +477,7 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
     });
   };
   auto stage = [&](int kt, auto first, auto loads, auto edge) {
-    if (kLate > 0 && kt + 1 < n_kt) {
+    if (kLate > 0 && kt + DA - 1 < n_kt) {  // none of them was left out
       wait_vmcnt<kLate>();
     } else {
       wait_vmcnt<0>();
@@ -442,6 +489,8 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
       constexpr bool kMul = decltype(gc)::value > 0 || !decltype(first)::value;
       group(kt, gc, std::bool_constant<kMul>{}, loads, edge);
     });
+    slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
+    slot_b = slot_b == SB - 1 ? 0 : slot_b + 1;
   };
   static_assert(KS % 2 == 0, "substep buffers alternate within a stage");
   using Zero = std::integral_constant<int, 0>;
@@ -471,6 +520,104 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
   if (n_kt > 0) {
 #pragma unroll
     for (int g = 0; g < NM; ++g) mfma(1, g);
+  }
+  epi.template apply<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane, lds);
+}
+
+// The same product for small wavefront tiles (64 x 64 and below), whose substep is too few MFMAs to
+// cover an LDS read: the fragments of a whole stage are in registers, and while stage kt - 1 is
+// multiplied substep by substep, the registers of each finished substep are refilled from stage kt.
+// A fragment then has three substeps of MFMAs to arrive in. One ring of S stages of both operands,
+// loaded S - 2 stages ahead: the slot that stage kt's loads fill was last read two barriers ago, so
+// the barrier waits for no fragment read.
+template <int BM, int BN, int WM, int WN, int S, class SrcA, class SrcB, class Epi>
+__device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int k_begin, int k_end,
+                                               int tm, int tn, Epi& epi, uint4* lds) {
+  constexpr int BK = 64, NW = WM * WN, KS = BK / 16, D = S - 2;
+  constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
+  static_assert(TM * 32 == WTM && TN * 32 == WTN, "wave tiles are multiples of 32");
+  static_assert(D >= 1, "a ring of at least three stages");
+  using LA = LdsTile<BK, false, BM>;
+  using LB = LdsTile<BK, false, BN>;
+  constexpr int kTileA = BM * LA::kRC, kStage = (BM + BN) * LA::kRC;
+  using TA = std::conditional_t<SrcA::kSegmented, DmaTileSeg<BM, NW, BK>, DmaTile<BM, NW, BK>>;
+  using TB = std::conditional_t<SrcB::kKMajor, DmaTileK<BN, NW, BK>, DmaTile<BN, NW, BK>>;
+  constexpr int kDma = TA::kPer + TB::kPer, NM = TM * TN, NR = TM + TN;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave / WN, wn = wave % WN;
+  TA la;
+  TB lb;
+  la.init(A, m0, wave, lane);
+  lb.init(B, n0, wave, lane);
+  epi.template prepare<TM, TN>(m0 + wm * WTM, n0 + wn * WTN, lane);
+  floatx16 acc[TM][TN];
+  epi.template start<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane);
+  const int n_kt = (k_end - k_begin + BK - 1) / BK;
+  auto load = [&](int kt, int q) {
+    uint4* st = lds + (kt % S) * kStage;
+    const int k0 = k_begin + kt * BK;
+    if (q < TA::kPer) la.issue_inside(A, m0, k0, st, wave, q);
+    else lb.issue_inside(B, n0, k0, st + kTileA, wave, q - TA::kPer);
+  };
+  const int arow = wm * WTM + lane % 32, brow = wn * WTN + lane % 32;
+  half8 af[KS][TM], bf[KS][TN];
+  auto read = [&](const uint4* st, int ks, int r) {
+    const int ch = ks * 2 + lane / 32;
+    if (r < TM) {
+      af[ks][r] = LA::frag(st, arow + r * 32, ch);
+    } else if constexpr (SrcB::kKMajor) {
+      bf[ks][r - TM] = frag_kmajor<BN>(st + kTileA, wn * WTN + (r - TM) * 32, ks, lane);
+    } else {
+      bf[ks][r - TM] = LB::frag(st + kTileA, brow + (r - TM) * 32, ch);
+    }
+  };
+  auto mfma = [&](int ks, int g) {
+    const int i = g / TN, j = g % TN;
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks][i], bf[ks][j], acc[i][j], 0, 0, 0);
+  };
+  static_for<D>([&](auto sc) {
+    constexpr int s = decltype(sc)::value;
+    if (s < n_kt) {
+#pragma unroll
+      for (int q = 0; q < kDma; ++q) load(s, q);
+    }
+  });
+  epi.template started<TM, TN>(acc);
+  auto stage = [&](int kt, auto first, auto loads) {
+    // the loads of stages kt + 1 .. kt + D - 1 may still be in flight when all were issued
+    if (D > 1 && kt + D - 1 < n_kt) wait_vmcnt<(D - 1) * kDma>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const uint4* st = lds + (kt % S) * kStage;
+    constexpr int kStep = NM > NR ? NM : NR;  // slots per substep
+    // substep s's slots multiply it and read substep s - 1 of the new stage
+    static_for<(KS + 1) * kStep>([&](auto sc) {
+      constexpr int slot = decltype(sc)::value, ks = slot / kStep, m = slot % kStep;
+      if constexpr (ks < KS && m < NM && !decltype(first)::value) mfma(ks, m);
+      if constexpr (ks > 0 && m < NR) read(st, ks - 1, m);
+      if constexpr (decltype(loads)::value) {
+        static_for<kDma>([&](auto qc) {
+          constexpr int q = decltype(qc)::value;
+          if constexpr ((2 * q + 1) * KS * kStep / (2 * kDma) == slot) load(kt + D, q);
+        });
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  if (n_kt > 0) {
+    if (D < n_kt) stage(0, std::true_type{}, std::true_type{});
+    else stage(0, std::true_type{}, std::false_type{});
+    int kt = 1;
+    for (; kt + D < n_kt; ++kt) stage(kt, std::false_type{}, std::true_type{});
+    for (; kt < n_kt; ++kt) stage(kt, std::false_type{}, std::false_type{});
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int g = 0; g < NM; ++g) mfma(ks, g);
   }
   epi.template apply<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane, lds);
 }

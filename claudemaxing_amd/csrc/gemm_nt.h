@@ -22,6 +22,7 @@ constexpr int kRowChunks = kBK / 8;  // 16-byte chunks per tile row
 struct RowMajor {
   static constexpr bool kChunkMajor = false;  // LDS tile layout (gemm_lds.h)
   static constexpr bool kKMajor = false;
+  static constexpr bool kSegmented = false;
   const _Float16* p;
   int64_t ld;
   int rows;   // valid rows
@@ -51,6 +52,7 @@ struct Tiled32 {
   static constexpr bool kChunkMajor = true;
   static constexpr int kChunkBytes = 512;  // between a row's neighbouring 8-column chunks
   static constexpr bool kKMajor = false;
+  static constexpr bool kSegmented = false;
   const _Float16* p;
   int rows;        // valid rows
   int k_len;       // columns
@@ -71,6 +73,28 @@ struct Tiled32 {
   }
 };
 
+// Up to three row-major arrays side by side along k, each with its own base and row stride: segment s
+// holds columns first[s] .. first[s + 1] - 1 (whole 64-column stages). The gradients of several
+// outputs of one input, contracted together.
+struct SegRows {
+  static constexpr bool kChunkMajor = false;
+  static constexpr bool kKMajor = false;
+  static constexpr bool kSegmented = true;
+  const _Float16* p[3];
+  int64_t ld[3];
+  int first[3];  // an unused segment's is past k_len
+  int rows;
+  int k_len;
+  // the address of (r, k) and the row stride there; k uniform over the wavefront
+  __device__ __forceinline__ const _Float16* at(int r, int k, int64_t& stride) const {
+    const bool s1 = k >= first[1], s2 = k >= first[2];
+    stride = s2 ? ld[2] : s1 ? ld[1] : ld[0];
+    const _Float16* base = s2 ? p[2] : s1 ? p[1] : p[0];
+    return base + static_cast<int64_t>(r) * stride + (k - (s2 ? first[2] : s1 ? first[1] : 0));
+  }
+  __device__ __forceinline__ bool k_inside(int) const { return true; }
+};
+
 // An NT operand stored transposed, [K][N] with N contiguous: element (row n, column k) of the
 // operand at p[k * ld + n]. The LM head reads its weight W [V][H] this way as the gradient GEMM's
 // B operand (rows = hidden units, K = vocabulary), so that no transposed copy of W is needed.
@@ -79,6 +103,7 @@ struct Tiled32 {
 struct KMajor {
   static constexpr bool kChunkMajor = false;
   static constexpr bool kKMajor = true;
+  static constexpr bool kSegmented = false;
   const _Float16* p;
   int64_t ld;  // elements between consecutive k
   int rows;    // valid n

@@ -325,23 +325,34 @@ __global__ __launch_bounds__(kThreads) void lora_fused_bwd1_kernel(Bwd1Jobs jobs
 // Backward-2 needs no sum across lanes (each input's gxd is a rank-16 sum): lane c of the
 // workgroup owns inputs 4 c .. 4 c + 3 of R token rows. Its 16 columns of fp16(A) (one 16-byte
 // read per rank, contiguous across the lanes) serve all R rows, and every row's dxb (or dx), x16
-// and mask nibble are loaded at once, so a workgroup waits for memory once. gxd sums the 16
+// and mask nibbles are loaded at once, so a workgroup waits for memory once. gxd sums the 16
 // rank products in rank order. MODE is 0 without dx, 1 for dx = dxb + term, 2 for dx += term (a
 // compile-time choice: a branch on it between the loads would make the compiler wait for each
-// row's loads in turn).
-template <int R, int MODE>
+// row's loads in turn). J adapters of one input (a block's q and v) add their terms in order, as one
+// launch after the other would: dx is written once, dxb and x16 are read once (1276 x 1536, two
+// adapters: 20.8 us as two launches in a captured step, 16.9 as one on cold caches).
+struct Bwd2Job {
+  const _Float16* ga16;
+  const float* A;
+  const uint8_t* bits;
+  _Float16* xd16;
+};
+constexpr int kMaxBwd2 = 2;
+struct Bwd2Jobs {
+  Bwd2Job j[kMaxBwd2];
+};
+
+template <int R, int MODE, int J>
 __global__ __launch_bounds__(kMaxK / 4) void lora_fused_bwd2_kernel(
-    const _Float16* __restrict__ dxb, const _Float16* __restrict__ ga16,
-    const float* __restrict__ A, const _Float16* __restrict__ x16,
-    const uint8_t* __restrict__ bits, float* __restrict__ dx, _Float16* __restrict__ xd16,
-    int T, int K, float scale_p) {
-  __shared__ half8 s_g[R][2];  // ga of the workgroup's rows
+    const _Float16* __restrict__ dxb, Bwd2Jobs jobs, const _Float16* __restrict__ x16,
+    float* __restrict__ dx, int T, int K, float scale_p) {
+  __shared__ half8 s_g[J][R][2];  // ga of the workgroup's rows
   const int c = threadIdx.x, K4 = K / 4, K8 = K / 8, t0 = blockIdx.x * R;
   const bool kok = c < K4;
   const int cc = kok ? c : K4 - 1;  // clamped column quad
   uint4 prior[R];  // the 4 fp16 of dxb in .x/.y, or the 4 fp32 of dx as it is (accumulating)
   uint2 xq[R];
-  uint32_t mb[R];
+  uint32_t mb[J][R];
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     const int64_t tc = min(t0 + i, T - 1);
@@ -355,56 +366,69 @@ __global__ __launch_bounds__(kMaxK / 4) void lora_fused_bwd2_kernel(
       prior[i] = make_uint4(0u, 0u, 0u, 0u);
     }
     xq[i] = *reinterpret_cast<const uint2*>(x16 + at);
-    mb[i] = bits[tc * K8 + cc / 2];
-  }
-  float4 ac[kR];  // fp32 A[r][4 c .. 4 c + 3], then its fp16 values
 #pragma unroll
-  for (int r = 0; r < kR; ++r)
-    ac[r] = *reinterpret_cast<const float4*>(A + static_cast<int64_t>(r) * K + 4 * cc);
+    for (int j = 0; j < J; ++j) mb[j][i] = jobs.j[j].bits[tc * K8 + cc / 2];
+  }
+  float4 ac[J][kR];  // fp32 A[r][4 c .. 4 c + 3], then its fp16 values
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+      ac[j][r] = *reinterpret_cast<const float4*>(jobs.j[j].A + static_cast<int64_t>(r) * K + 4 * cc);
   if (threadIdx.x < 2 * R) {
     const int i = threadIdx.x / 2, h = threadIdx.x % 2;
-    s_g[i][h] = *reinterpret_cast<const half8*>(
-        ga16 + static_cast<int64_t>(min(t0 + i, T - 1)) * kR + 8 * h);
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      s_g[j][i][h] = *reinterpret_cast<const half8*>(
+          jobs.j[j].ga16 + static_cast<int64_t>(min(t0 + i, T - 1)) * kR + 8 * h);
   }
   __syncthreads();
   if (!kok) return;  // no barrier below
 #pragma unroll
-  for (int r = 0; r < kR; ++r) {
-    ac[r].x = static_cast<float>(h16(ac[r].x));
-    ac[r].y = static_cast<float>(h16(ac[r].y));
-    ac[r].z = static_cast<float>(h16(ac[r].z));
-    ac[r].w = static_cast<float>(h16(ac[r].w));
-  }
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      ac[j][r].x = static_cast<float>(h16(ac[j][r].x));
+      ac[j][r].y = static_cast<float>(h16(ac[j][r].y));
+      ac[j][r].z = static_cast<float>(h16(ac[j][r].z));
+      ac[j][r].w = static_cast<float>(h16(ac[j][r].w));
+    }
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     if (t0 + i >= T) break;
-    const half8 g0 = s_g[i][0], g1 = s_g[i][1];
-    float gx[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      const float g = static_cast<float>(r < 8 ? g0[r] : g1[r - 8]);
-      gx[0] += g * ac[r].x;
-      gx[1] += g * ac[r].y;
-      gx[2] += g * ac[r].z;
-      gx[3] += g * ac[r].w;
-    }
-    const uint32_t nib = (mb[i] >> (4 * (c & 1))) & 0xfu;
     const half4 db = __builtin_bit_cast(half4, make_uint2(prior[i].x, prior[i].y));
     const half4 xv = __builtin_bit_cast(half4, xq[i]);
     const uint32_t dold[4] = {prior[i].x, prior[i].y, prior[i].z, prior[i].w};
     float o[4];
-    half4 xo;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool kept = (nib >> e) & 1u;
-      const float gl = kept ? static_cast<float>(h16(gx[e])) * scale_p : 0.0f;
-      o[e] = (MODE == 1 ? static_cast<float>(db[e]) : __uint_as_float(dold[e])) + gl;
-      xo[e] = h16(kept ? static_cast<float>(xv[e]) * scale_p : 0.0f);
-    }
+    for (int e = 0; e < 4; ++e)
+      o[e] = MODE == 1 ? static_cast<float>(db[e]) : __uint_as_float(dold[e]);
     const int64_t at = static_cast<int64_t>(t0 + i) * K + 4 * c;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const half8 g0 = s_g[j][i][0], g1 = s_g[j][i][1];
+      float gx[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < kR; ++r) {
+        const float g = static_cast<float>(r < 8 ? g0[r] : g1[r - 8]);
+        // the product of two fp16 values is exact in fp32: one rounding either way
+        gx[0] = __builtin_fmaf(g, ac[j][r].x, gx[0]);
+        gx[1] = __builtin_fmaf(g, ac[j][r].y, gx[1]);
+        gx[2] = __builtin_fmaf(g, ac[j][r].z, gx[2]);
+        gx[3] = __builtin_fmaf(g, ac[j][r].w, gx[3]);
+      }
+      const uint32_t nib = (mb[j][i] >> (4 * (c & 1))) & 0xfu;
+      half4 xo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool kept = (nib >> e) & 1u;
+        o[e] += kept ? static_cast<float>(h16(gx[e])) * scale_p : 0.0f;
+        xo[e] = h16(kept ? static_cast<float>(xv[e]) * scale_p : 0.0f);
+      }
+      *reinterpret_cast<half4*>(jobs.j[j].xd16 + at) = xo;
+    }
     if constexpr (MODE != 0)
       *reinterpret_cast<float4*>(dx + at) = make_float4(o[0], o[1], o[2], o[3]);
-    *reinterpret_cast<half4*>(xd16 + at) = xo;
   }
 }
 
@@ -429,7 +453,21 @@ int quad_rows(int64_t T) {
   return r;
 }
 
-// Token rows per tile: 16, or fewer when 16-row tiles would leave CUs idle.
+// The same for two adapters in one launch, whose registers leave a CU one workgroup at a time: the
+// fewest of 1, 2, 4, 8 that make one round of them (more rows are read per workgroup, but a second
+// round costs a memory round trip: 1276 rows 21.5 us in two rounds of 4, 19.0 in one of 8; 300 rows
+// 10.0 us with 2 rows, 17.1 with 8).
+constexpr int kPairRows = 8;
+int quad_rows_pair(int64_t T) {
+  int r = 1;
+  while (r < kPairRows && (T + r - 1) / r > kCUs) r *= 2;
+  return r;
+}
+
+// Token rows per tile, for T rows over all adapters of the launch: 16, or fewer when 16-row tiles
+// would leave CUs idle. A CU holds one workgroup of the widest forward at a time, so the tiles of all
+// adapters together are one round (q and v at 1276 tokens: 10 rows, 19.8 us forward; 5 rows, two
+// rounds, 26.8).
 int tile_rows(int64_t T) {
   const int64_t r = (T + kCUs - 1) / kCUs;
   return static_cast<int>(std::min<int64_t>(kTileRows, std::max<int64_t>(1, r)));
@@ -477,7 +515,7 @@ bool fwd_job_ok(const float* x, const uint8_t* keep, const float* weight_a, cons
 
 int launch_fwd(const float* x, const FwdJobs& jobs, int n_jobs, int max_n, int64_t T, int K,
                float scale_p, float scaling, hipStream_t s) {
-  const int rows = tile_rows(T);
+  const int rows = tile_rows(T * n_jobs);
   dim3 grid = tile_grid(T, rows);
   grid.y = n_jobs;
   CM_LORA_SK_SWITCH(steps_bound(K), SK, CM_LORA_SN_SWITCH(tiles_bound(max_n), SN, {
@@ -496,7 +534,7 @@ bool bwd1_job_ok(const float* grad, const float* weight_b, const void* gbase16, 
 
 int launch_bwd1(const Bwd1Jobs& jobs, int n_jobs, int max_n, int64_t T, float scaling,
                 hipStream_t s) {
-  const int rows = tile_rows(T);
+  const int rows = tile_rows(T * n_jobs);
   dim3 grid = tile_grid(T, rows);
   grid.y = n_jobs;
   CM_LORA_SK_SWITCH(steps_bound(max_n), SN, {
@@ -580,29 +618,66 @@ extern "C" int cm_lora_fused_bwd1_multi(int64_t T, int rank, float scaling, int 
   return launch_bwd1(jobs, n_jobs, max_n, T, scaling, static_cast<hipStream_t>(stream));
 }
 
+namespace {
+
+bool bwd2_job_ok(const void* ga16, const float* weight_a, const uint8_t* bits, const void* xd16) {
+  return ga16 && weight_a && bits && xd16 && aligned(ga16, 16) && aligned(weight_a, 16) &&
+         aligned(xd16, 8);
+}
+
+template <int J>
+int launch_bwd2(const void* dxb16, const Bwd2Jobs& jobs, const void* x16, float* dx, int64_t T, int K,
+                float scale_p, hipStream_t s) {
+  const int mode = !dx ? 0 : dxb16 ? 1 : 2;
+  const int R = J == 1 ? quad_rows(T) : quad_rows_pair(T);
+  const dim3 grid(static_cast<unsigned>((T + R - 1) / R)), block((K / 4 + 63) / 64 * 64);
+  CM_LORA_J_SWITCH(R, RW, {
+    constexpr int RR = J == 1 || RW < kPairRows ? RW : kPairRows;
+    const auto kernel = mode == 0   ? lora_fused_bwd2_kernel<RR, 0, J>
+                        : mode == 1 ? lora_fused_bwd2_kernel<RR, 1, J>
+                                    : lora_fused_bwd2_kernel<RR, 2, J>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, static_cast<const _Float16*>(dxb16), jobs,
+                       static_cast<const _Float16*>(x16), dx, static_cast<int>(T), K, scale_p);
+  });
+  return cm::launch_status();
+}
+
+}  // namespace
+
 extern "C" int cm_lora_fused_bwd2(const void* dxb16, const void* ga16, const float* weight_a,
                                   const void* x16, const uint8_t* bits, float* dx, void* xd16,
                                   int64_t T, int K, int rank, float scale_p, void* stream) {
   CM_CHECK_ARG(rank == kR && T >= 0 && K > 0 && K % 8 == 0 && K <= kMaxK);
   if (T == 0) return 0;
   CM_CHECK_ARG(T <= 0x7fffffff / 2);
-  CM_CHECK_ARG(ga16 && weight_a && x16 && bits && xd16);
-  CM_CHECK_ARG((!dx || ((!dxb16 || aligned(dxb16, 8)) && aligned(dx, 16))) && aligned(ga16, 16) &&
-               aligned(weight_a, 16) && aligned(x16, 8) && aligned(xd16, 8));
+  CM_CHECK_ARG(x16 && aligned(x16, 8) && bwd2_job_ok(ga16, weight_a, bits, xd16));
+  CM_CHECK_ARG(!dx || ((!dxb16 || aligned(dxb16, 8)) && aligned(dx, 16)));
+  Bwd2Jobs jobs{};
+  jobs.j[0] = Bwd2Job{static_cast<const _Float16*>(ga16), weight_a, bits,
+                      static_cast<_Float16*>(xd16)};
+  return launch_bwd2<1>(dxb16, jobs, x16, dx, T, K, scale_p, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int cm_lora_fused_bwd2_multi(const void* dxb16, const void* x16, float* dx, int64_t T,
+                                        int K, int rank, float scale_p, int n_jobs,
+                                        const void* const* ga16, const float* const* weight_a,
+                                        const uint8_t* const* bits, void* const* xd16,
+                                        void* stream) {
+  CM_CHECK_ARG(rank == kR && T >= 0 && K > 0 && K % 8 == 0 && K <= kMaxK);
+  CM_CHECK_ARG(n_jobs >= 1 && n_jobs <= kMaxBwd2 && ga16 && weight_a && bits && xd16);
+  if (T == 0) return 0;
+  CM_CHECK_ARG(T <= 0x7fffffff / 2);
+  CM_CHECK_ARG(x16 && aligned(x16, 8));
+  CM_CHECK_ARG(!dx || ((!dxb16 || aligned(dxb16, 8)) && aligned(dx, 16)));
+  Bwd2Jobs jobs{};
+  for (int i = 0; i < n_jobs; ++i) {
+    CM_CHECK_ARG(bwd2_job_ok(ga16[i], weight_a[i], bits[i], xd16[i]));
+    jobs.j[i] = Bwd2Job{static_cast<const _Float16*>(ga16[i]), weight_a[i], bits[i],
+                        static_cast<_Float16*>(xd16[i])};
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int mode = !dx ? 0 : dxb16 ? 1 : 2;
-  const int R = quad_rows(T);
-  const dim3 grid(static_cast<unsigned>((T + R - 1) / R)), block((K / 4 + 63) / 64 * 64);
-  CM_LORA_J_SWITCH(R, RR, {
-    const auto kernel = mode == 0   ? lora_fused_bwd2_kernel<RR, 0>
-                        : mode == 1 ? lora_fused_bwd2_kernel<RR, 1>
-                                    : lora_fused_bwd2_kernel<RR, 2>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, static_cast<const _Float16*>(dxb16),
-                       static_cast<const _Float16*>(ga16), weight_a,
-                       static_cast<const _Float16*>(x16), bits, dx, static_cast<_Float16*>(xd16),
-                       static_cast<int>(T), K, scale_p);
-  });
-  return cm::launch_status();
+  return n_jobs == 1 ? launch_bwd2<1>(dxb16, jobs, x16, dx, T, K, scale_p, s)
+                     : launch_bwd2<2>(dxb16, jobs, x16, dx, T, K, scale_p, s);
 }
 
 // ---------------------------------------------------------------------------------------------

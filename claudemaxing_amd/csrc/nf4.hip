@@ -527,3 +527,19 @@ extern "C" int cm_nf4_dequant_group(const cm_nf4_weight* w, int n_w, void* const
   }
 #undef CM_NF4_GROUP
 }
+
+extern "C" int cm_nf4_expand_rows(const cm_nf4_weight* w, int n_w, void* out, int out_dtype,
+                                  void* stream) {
+  CM_CHECK_ARG(n_w >= 0 && n_w <= kGroupMax);
+  if (n_w == 0) return 0;
+  CM_CHECK_ARG(w && out);
+  const int size = cm::dtype_size(out_dtype);
+  void* outs[kGroupMax];
+  int64_t at = 0;
+  for (int i = 0; i < n_w; ++i) {
+    CM_CHECK_ARG(w[i].rows >= 0 && w[i].cols >= 0);
+    outs[i] = static_cast<char*>(out) + at * size;
+    at += w[i].rows * w[i].cols;
+  }
+  return cm_nf4_dequant_group(w, n_w, outs, out_dtype, stream);
+}

@@ -257,6 +257,44 @@ def nf4_linear_bwd(grads, pairs, dx_dtype=torch.float16):
     return dx.view(*grads[0].shape[:-1], k)
 
 
+def expand_rows(pairs):
+    """The fp16 weights of `pairs` one under another, [sum N_i, K], expanded in one launch."""
+    w = torch.empty(sum(int(st.shape[0]) for _, st in pairs), int(pairs[0][1].shape[1]),
+                    dtype=torch.float16, device=pairs[0][0].device)
+    _lib.call("cm_nf4_expand_rows", _plain_weights(pairs)[0], len(pairs), w.data_ptr(), _lib.F16,
+              _lib.stream(w.device))
+    return w
+
+
+def linear_rows_fwd(x16, w, sizes, biases):
+    """[x16 @ W_i.T (+ b_i)] in fp16 for the layers W_i [N_i, K] stacked in w (expand_rows), at most
+    three, in one launch (cm_linear_f16_fwd); N_i and K multiples of 64, biases fp16 or None."""
+    k, n = w.shape[1], len(sizes)
+    x2 = _rows16(x16, k)
+    m = x2.shape[0]
+    outs = [torch.empty(m, s, dtype=torch.float16, device=x2.device) for s in sizes]
+    biases = [None if b is None else b.to(torch.float16).contiguous() for b in biases]
+    P, L = ctypes.c_void_p * n, ctypes.c_int64 * n
+    _lib.call("cm_linear_f16_fwd", x2.data_ptr(), x2.stride(0), m, k, w.data_ptr(), n,
+              (ctypes.c_int * n)(*sizes), P(*[_lib.ptr(b) for b in biases]),
+              P(*[o.data_ptr() for o in outs]), L(*sizes), _lib.stream(x2.device))
+    return [o.view(*x16.shape[:-1], s) for o, s in zip(outs, sizes)]
+
+
+def linear_rows_bwd(grads, w, sizes):
+    """sum_i grads_i @ W_i in fp16, rounded once, for the layers stacked in w, in one launch
+    (cm_linear_f16_bwd)."""
+    k, n = w.shape[1], len(sizes)
+    g2 = [_rows16(g, s) for g, s in zip(grads, sizes)]
+    m = g2[0].shape[0]
+    dx = torch.empty(m, k, dtype=torch.float16, device=w.device)
+    P, L = ctypes.c_void_p * n, ctypes.c_int64 * n
+    _lib.call("cm_linear_f16_bwd", P(*[g.data_ptr() for g in g2]), L(*[g.stride(0) for g in g2]), m,
+              n, (ctypes.c_int * n)(*sizes), w.data_ptr(), k, dx.data_ptr(), k,
+              _lib.stream(w.device))
+    return dx.view(*grads[0].shape[:-1], k)
+
+
 class MatMulNF4(torch.autograd.Function):
     """x @ W.T (+ bias) for a frozen NF4 weight W [out, in], computed in `compute` dtype (x's
     own when None); an optional frozen bias in that dtype. An fp32 x is taken through the fp16

@@ -21,7 +21,7 @@
 extern "C" {
 #endif
 
-#define CM_ABI_VERSION 9
+#define CM_ABI_VERSION 10
 
 /* Element types of tensor arguments. */
 typedef enum {
@@ -100,6 +100,19 @@ int cm_gemm_f32_add(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, 
 int cm_gemm_f32_kb(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, int K0,
                    const void* a1, int64_t lda1, const void* b1, int64_t ldb1, int K1, int M,
                    int N, float* out, void* workspace, int64_t ws_bytes, void* stream);
+
+/* fp16 linear layers that share an input, on expanded weights: w is the layers' weights [N_i, K] one
+ * under another (sum N_i rows of K), n_out <= 3. Forward: out_i [M, N_i] (row stride ldo_i) =
+ * fp16(x W_i^T (+ bias_i)), x [M, K] (row stride ldx); bias may be null, and so may each bias_i.
+ * Backward: dx [M, K] (row stride ldx) = fp16(sum_i grad_i W_i), grad_i [M, N_i] (row stride ldg_i).
+ * All fp16 with fp32 sums, rounded once; K and every N_i multiples of 64, row strides of 8, pointers
+ * (but the biases) 16-byte aligned. Nothing is allocated and no workspace is needed. The reference
+ * runs each layer as a dequantization and a GEMM of its own (solution/nf4.py:102-130). */
+int cm_linear_f16_fwd(const void* x, int64_t ldx, int64_t M, int K, const void* w, int n_out,
+                      const int* N, const void* const* bias, void* const* out, const int64_t* ldo,
+                      void* stream);
+int cm_linear_f16_bwd(const void* const* grad, const int64_t* ldg, int64_t M, int n_in,
+                      const int* N, const void* w, int K, void* dx, int64_t ldx, void* stream);
 
 /* The same expansion written transposed, fp16 only: out[c][r] = W[r][c] for the weight W
  * [rows, cols] (rows a multiple of 64, cols of 128; packed 4-byte, out 16-byte aligned), the values
@@ -473,6 +486,13 @@ int cm_lora_fused_bwd1_multi(int64_t T, int rank, float scaling, int n_jobs,
 int cm_lora_fused_bwd2(const void* dxb16, const void* ga16, const float* weight_a,
                        const void* x16, const uint8_t* bits, float* dx, void* xd16, int64_t T,
                        int K, int rank, float scale_p, void* stream);
+/* cm_lora_fused_bwd2 for up to two adapters on one input x16 in one launch: dx = dxb16 (or dx as it
+ * is, without dxb16) + the adapters' terms, added in order; the same bits as one call per adapter, the
+ * first with dxb16. */
+int cm_lora_fused_bwd2_multi(const void* dxb16, const void* x16, float* dx, int64_t T, int K,
+                             int rank, float scale_p, int n_jobs, const void* const* ga16,
+                             const float* const* weight_a, const uint8_t* const* bits,
+                             void* const* xd16, void* stream);
 
 /* ------------------------------------------------------------------------------------------ */
 /* NF4 weights expanded inside an fp16 matrix-core GEMM (the fp16 weight is never written to
@@ -552,6 +572,9 @@ int64_t cm_nf4_linear_workspace_bytes(int64_t m, const cm_nf4_weight* w, int n_w
  */
 int cm_nf4_dequant_group(const cm_nf4_weight* w, int n_w, void* const* out, int out_dtype,
                          void* stream);
+/* cm_nf4_dequant_group with the outputs one under another in out: weight i's rows after weight
+ * i - 1's (the [sum rows, cols] operand of cm_linear_f16_fwd / _bwd for weights of one width). */
+int cm_nf4_expand_rows(const cm_nf4_weight* w, int n_w, void* out, int out_dtype, void* stream);
 
 /* ---- On-box peak probes (measurement only; no counterpart in the reference) ----------------
  * The roofline denominators as this board attains them, which bench.py reports beside the

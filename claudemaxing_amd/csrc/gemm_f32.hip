@@ -33,9 +33,11 @@ constexpr int kThreads = kWM * kWN * cm::kWave;
 constexpr int kMaxSlices = 16;
 constexpr int kCUs = 256;
 
-// The fp32 partial tile of one K-slice, rows past M and columns past N dropped.
+// The fp32 partial tile of one K-slice, rows past M and columns past N dropped; with `residual` (the
+// one slice of an unsplit contraction), residual + the tile.
 struct EpiSlice {
-  float* out;  // [M, N] slice of the workspace
+  float* out;  // [M, N]: a slice of the workspace, or the result
+  const float* residual;
   int M, N;
   template <int TM, int TN>
   __device__ __forceinline__ void prepare(int, int, int) {}
@@ -57,7 +59,9 @@ struct EpiSlice {
 #pragma unroll
         for (int nt = 0; nt < TN; ++nt) {
           const int col = nb + nt * 32 + lane % 32;
-          if (col < N) out[static_cast<int64_t>(row) * N + col] = acc[mt][nt][r];
+          if (col >= N) continue;
+          const int64_t at = static_cast<int64_t>(row) * N + col;
+          out[at] = residual != nullptr ? residual[at] + acc[mt][nt][r] : acc[mt][nt][r];
         }
       }
   }
@@ -72,7 +76,8 @@ struct Pairs {
 
 template <bool KB>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int remap, float* ws,
-                                                               int M, int N) {
+                                                               const float* residual, int M,
+                                                               int N) {
   __shared__ uint4 lds[(kSA * kBM + kSB * kBN) * (kBK / 8)];
   int tm, tn, s;
   cm::gemm::tile_of_block_2d((N + kBN - 1) / kBN, remap, tm, tn, s);
@@ -80,7 +85,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int rema
   const int k_begin = sq * p.k_slice[q];
   // an empty slice still writes its (zero) partial tile, which the sum then reads
   const int k_end = max(k_begin, min(p.a[q].k_len, k_begin + p.k_slice[q]));
-  EpiSlice epi{ws + static_cast<int64_t>(s) * M * N, M, N};
+  EpiSlice epi{ws + static_cast<int64_t>(s) * M * N, residual, M, N};
   if constexpr (KB) {
     if (q == 0) {
       cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[0], p.bk[0], k_begin, k_end, tm,
@@ -178,7 +183,7 @@ int gemm_f32_impl(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, in
                   void* stream, bool b_kmajor = false) {
   CM_CHECK_ARG(shape_ok(M, N, K0, K1));
   if (M == 0 || N == 0) return 0;
-  CM_CHECK_ARG(a0 && b0 && out && workspace && (K1 == 0 || (a1 && b1)));
+  CM_CHECK_ARG(a0 && b0 && out && (K1 == 0 || (a1 && b1)));
   // B's rows: K of them of N values when k-major (N a multiple of 8: whole 16-byte chunks), else
   // N rows of K
   const int64_t b_row = b_kmajor ? N : 0;
@@ -191,7 +196,10 @@ int gemm_f32_impl(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, in
                (K1 == 0 || (al16(a1) && al16(b1))) && (!residual || al16(residual)));
   CM_CHECK_ARG(static_cast<int64_t>(M) * N % 4 == 0);
   const Plan pl = plan_for(M, N, K0, K1);
-  CM_CHECK_ARG(ws_bytes >= static_cast<int64_t>(pl.total()) * M * N * 4);
+  // one slice: the tiles are the result, without a sum, and the workspace may be left out
+  const bool direct = pl.total() == 1;
+  CM_CHECK_ARG((direct && ws_bytes == 0) ||
+               (workspace && ws_bytes >= static_cast<int64_t>(pl.total()) * M * N * 4));
   Pairs p{};
   p.a[0] = RowMajor{static_cast<const _Float16*>(a0), lda0, M, K0};
   p.b[0] = RowMajor{static_cast<const _Float16*>(b0), ldb0, N, K0};
@@ -205,14 +213,16 @@ int gemm_f32_impl(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, in
   const int tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
   const int remap = (tiles * pl.total()) % 8 == 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  float* ws = static_cast<float*>(workspace);
+  float* ws = direct ? out : static_cast<float*>(workspace);
+  const float* res = direct ? residual : nullptr;
   if (b_kmajor) {
     hipLaunchKernelGGL(gemm_f32_kernel<true>, dim3(tiles, pl.total()), dim3(kThreads), 0, s, p,
-                       remap, ws, M, N);
+                       remap, ws, res, M, N);
   } else {
     hipLaunchKernelGGL(gemm_f32_kernel<false>, dim3(tiles, pl.total()), dim3(kThreads), 0, s, p,
-                       remap, ws, M, N);
+                       remap, ws, res, M, N);
   }
+  if (direct) return cm::launch_status();
   const int64_t n4 = static_cast<int64_t>(M) * N / 4;
   hipLaunchKernelGGL(gemm_f32_sum, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, s,
                      reinterpret_cast<const float4*>(ws), pl.total(), n4,

@@ -24,6 +24,20 @@ def split_k_pays(m, n, k):
     return tiles < 128 and k >= 4096
 
 
+def kmajor_pays(m, n, k):
+    """Whether an fp32-output product with a k-major weight (dx = y W) is worth the split-K GEMM: where
+    split_k_pays, and on larger outputs while its tiles and slices fill one round of the 256 CUs to
+    nearly three quarters. There the product itself takes about the library's time, and what pays is
+    the merged weight it allows: one gate/up product along rows instead of two against transposed
+    copies. 1536 x 8960 MLP, recomputation + dx, us, merged / transposed: 4096 tokens (128 tiles x 2)
+    408 / 498, 6144 (192) 621 / 652, 8192 (256) 778 / 823; 5000 (160 tiles, 63%) 565 / 536; 2500
+    tokens of 3584 x 18944 (190) 1310 / 1775."""
+    if split_k_pays(m, n, k):
+        return True
+    tiles = -(-m // 256) * -(-n // 192)
+    return k >= 4096 and tiles <= 256 and tiles * (256 // tiles) >= 184
+
+
 def gemm_f32_supported(m, n, *pairs, b_kmajor=False):
     """Whether cm_gemm_f32 takes these operands: fp16, row-major with 16-byte aligned rows,
     contractions multiples of 8, on the GPU, and an output of a multiple of 4 elements (with
@@ -60,6 +74,8 @@ def gemm_f32(*pairs, out=None, residual=None, b_kmajor=False):
     ws_bytes = int(_lib.load().cm_gemm_f32_workspace_bytes(m, n, k0, k1))
     if ws_bytes < 0:
         raise RuntimeError("cm_gemm_f32_workspace_bytes: invalid shape")
+    if ws_bytes == 4 * m * n:  # one slice: written straight to the result
+        ws_bytes = 0
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=a0.device)
     common = (a0.data_ptr(), a0.stride(0), b0.data_ptr(), b0.stride(0), k0, _lib.ptr(a1),
               a1.stride(0) if rest else 0, _lib.ptr(b1), b1.stride(0) if rest else 0, k1, m, n)

@@ -78,8 +78,9 @@ int cm_lora_weight_grads(const void* const* w, const int64_t* ldw, const int* d,
  * bitsandbytes' gemm_4bit falls back to) and the MLP input gradient dgate Wg + dup Wu (autograd
  * of the two projections, the reference's MLPInputRecompute backward). Work split into K-slices
  * whose fp32 partial tiles go to `workspace` (cm_gemm_f32_workspace_bytes bytes) and are added in
- * slice order: deterministic, sums in fp32 (their order differs from a library GEMM's). All
- * pointers 16-byte aligned, M * N a multiple of 4. */
+ * slice order: deterministic, sums in fp32 (their order differs from a library GEMM's). A
+ * contraction that stays in one slice (the query gives M * N * 4) is written straight to out and may
+ * be given no workspace (null, 0 bytes). All pointers 16-byte aligned, M * N a multiple of 4. */
 int64_t cm_gemm_f32_workspace_bytes(int M, int N, int K0, int K1);
 int cm_gemm_f32(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, int K0,
                 const void* a1, int64_t lda1, const void* b1, int64_t ldb1, int K1, int M, int N,

@@ -3,7 +3,7 @@ which products take them, and that anything they cannot take falls back."""
 
 import torch
 
-from claudemaxing_amd.gemm import gemm_f32_supported, split_k_pays
+from claudemaxing_amd.gemm import gemm_f32_supported, kmajor_pays, split_k_pays
 from claudemaxing_amd.lora import _weight_grads
 
 
@@ -14,6 +14,16 @@ def test_split_k_pays_for_narrow_long_contractions():
     assert not split_k_pays(1276, 1536, 1536)
     assert not split_k_pays(1276, 8960, 1536)
     assert not split_k_pays(32768, 1536, 8960)  # 128 x 8 tiles fill the chip by themselves
+
+
+def test_kmajor_pays_where_tiles_and_slices_fill_a_round():
+    k = 2 * 8960
+    assert kmajor_pays(1276, 1536, k)  # as split_k_pays
+    assert kmajor_pays(4096, 1536, k)  # 128 tiles x 2 slices
+    assert not kmajor_pays(5000, 1536, k)  # 160 tiles of 256 CUs
+    assert kmajor_pays(5888, 1536, k) and not kmajor_pays(5632, 1536, k)  # 184 and 176 tiles
+    assert kmajor_pays(8192, 1536, k) and not kmajor_pays(8193, 1536, k)  # 256 and 264
+    assert not kmajor_pays(8192, 1536, 1536)  # a short contraction
 
 
 def test_cpu_operands_are_not_taken():

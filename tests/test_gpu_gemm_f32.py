@@ -121,3 +121,24 @@ def test_kmajor_b_row_stride(dev):
     out = gemm_f32((a, b), b_kmajor=True)
     assert torch.equal(out, gemm_f32((a, bt)))
     assert not gemm_f32_supported(96, 60, (a, b[:, :60]), b_kmajor=True)  # N % 8
+
+
+@pytest.mark.parametrize("m,n,k0,k1", [(4096, 1536, 4104, 4104), (6001, 1544, 4096, 0), (255, 200, 64, 0),
+                                       (257, 8, 72, 0)])
+def test_one_slice_is_written_straight(m, n, k0, k1, dev):
+    """Contractions that are not split (enough tiles, or too few stages) go to the result without
+    partial sums: row-major and k-major B alike, with a residual too, edge tiles in m and n."""
+    banner(f"gemm_f32 unsplit m={m} n={n} k0={k0} k1={k1}")
+    ref, rm, kb = 0, [], []
+    for i, k in enumerate((k0, k1)):
+        if k:
+            a, bt = _pair(m, n, k, dev, 11 + i)
+            rm.append((a, bt))
+            kb.append((a, bt.t().contiguous()))
+            ref = ref + a.double() @ bt.t().double()
+    out = gemm_f32(*rm)
+    torch.cuda.synchronize()
+    _check(out, ref, "unsplit")
+    assert torch.equal(out, gemm_f32(*kb, b_kmajor=True))
+    res = torch.randn(m, n, device=dev, generator=torch.Generator(device=dev).manual_seed(13))
+    assert torch.equal(gemm_f32(*rm, residual=res), res + out)

@@ -273,3 +273,21 @@ def test_patched_nf4_mlp_matches_the_original(dev, monkeypatch):
                                atol=2e-3 * float(ref.abs().max()))
     torch.testing.assert_close(xn.grad, xr.grad, rtol=2e-3,
                                atol=2e-3 * float(xr.grad.abs().max()))
+
+
+@pytest.mark.gpu
+def test_merged_route_with_an_unsplit_input_gradient(dev, monkeypatch):
+    """5883 tokens of a 1600-wide layer: 23 x 9 output tiles, one slice each (the input gradient is
+    written without partial sums, its last tiles reaching past the tokens and the width)."""
+    tokens, in_f = 5883, 1600
+    banner(f"MLPInputRecompute merged, unsplit, tokens={tokens}")
+    gp, upp = (nf4_layer(F, in_f, i, torch.float16, dev) for i in (1, 2))
+    g = torch.Generator().manual_seed(3)
+    x = (torch.randn(tokens, in_f, generator=g) * 2).to(dev)
+    grad = torch.randn(tokens, F, generator=g).to(dev)
+    out, dx, taken = routed(x, gp, upp, grad, monkeypatch)
+    assert taken == ["_dx_merged"], taken
+    s_out, s_dx = stock(x, gp, upp, grad)
+    r_out, r_dx = fp32_reference(x, oracle_weight(gp), oracle_weight(upp), grad)
+    check("unsplit output", out, s_out, r_out, 2e-3)
+    check("unsplit input gradient", dx, s_dx, r_dx, 2e-3)

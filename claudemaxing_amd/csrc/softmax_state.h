@@ -33,20 +33,6 @@ struct SoftmaxState {
     return SoftmaxState{-__builtin_huge_valf(), 0.0f, 0.0f, int64_t{0x7fffffffffffffff}};
   }
 
-  // Add logit z at column c; columns must arrive in increasing order per state.
-  __device__ __forceinline__ void push(float z, int64_t c) {
-    if (z > max) {
-      const float r = exp_f(max - z);  // 0 while the state is empty
-      sum *= r;
-      dot *= r;
-      max = z;
-      best = c;
-    }
-    const float e = exp_f(z - max);
-    sum += e;
-    dot += e * z;
-  }
-
   __device__ __forceinline__ void merge(const SoftmaxState& o) {
     if (o.max == -__builtin_huge_valf()) return;
     if (max == -__builtin_huge_valf()) {
@@ -71,25 +57,6 @@ __device__ __forceinline__ SoftmaxState shfl_xor_state(const SoftmaxState& s, in
   o.dot = __shfl_xor(s.dot, off, kWave);
   o.best = __shfl_xor(s.best, off, kWave);
   return o;
-}
-
-__device__ __forceinline__ SoftmaxState wave_merge(SoftmaxState s) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s.merge(shfl_xor_state(s, off));
-  return s;
-}
-
-// Merge the states of all lanes of a THREADS-lane workgroup; every lane gets the result.
-template <int THREADS>
-__device__ __forceinline__ SoftmaxState block_merge(SoftmaxState s, SoftmaxState* part) {
-  s = wave_merge(s);
-  const int wave = threadIdx.x / kWave;
-  if (threadIdx.x % kWave == 0) part[wave] = s;
-  __syncthreads();
-  SoftmaxState r = part[0];
-#pragma unroll
-  for (int i = 1; i < THREADS / kWave; ++i) r.merge(part[i]);
-  return r;
 }
 
 }  // namespace cm

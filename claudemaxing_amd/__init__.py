@@ -19,7 +19,7 @@ from .swiglu_recompute import patch_qwen2_mlp_recompute
 
 def apply():
     """Apply the patches in the reference's order (solution/__init__.py:25-34), with two of this
-    package's own before the last (q/k/v as one fused NF4 GEMM, and the decoder layer's residual
+    package's own before the last (q/k/v as one product, and the decoder layer's residual
     adds inside its norms: the same arithmetic in fewer launches). The last one,
     the attention patch (attention.py, `patch_qwen2_grouped_sdpa`), routes the packed batch of
     the fused training forward to the native packed causal attention kernels. Other boolean
@@ -32,6 +32,6 @@ def apply():
     patch_qwen2_rope()  # rotary embedding, q and k in one launch
     patch_bnb_nf4_dequant()  # NF4 dequantization (when bitsandbytes is installed)
     patch_peft_lora_4bit()  # LoRA branch with a packed dropout mask (when peft is installed)
-    patch_qwen2_fused_qkv()  # q/k/v of NF4 + LoRA blocks as one fused NF4 GEMM each way
+    patch_qwen2_fused_qkv()  # q/k/v of NF4 + LoRA blocks as one product each way
     patch_qwen2_decoder_residual()  # the decoder layer's residual adds inside its norms
     patch_qwen2_grouped_sdpa()  # causal attention of the packed batch

@@ -66,19 +66,30 @@ __device__ __forceinline__ int row_of_block(const Rows& rows, int b) {
   return r;
 }
 
+// Whether padded block b lies in a row (real tokens s0 .. s1 - 1, padded positions p0 .. p1 - 1) that
+// the kernels may work on: the block inside the row's padded positions, these inside the image's pend
+// (at most the launch's n_pad), whole blocks, and room for the row's real tokens, which are among the
+// launch's n_tokens. A kernel then reads and writes positions p0 .. p1 - 1 and tokens s0 .. s1 - 1 only,
+// whatever the image holds otherwise.
+__device__ __forceinline__ bool row_ok(int b, int s0, int s1, int p0, int p1, int pend,
+                                       int n_tokens) {
+  const int len = s1 - s0;
+  return s0 >= 0 && len >= 0 && s1 <= n_tokens && p0 % kBlk == 0 && p0 <= b * kBlk &&
+         b * kBlk < p1 && p1 <= pend && len <= p1 - p0;
+}
+
 // Whether padded block b of a launch for n_tokens tokens and n_pad padded positions has work:
 // the image is consistent with the launch (a row count the struct holds, n_tokens tokens, a
-// padded count within n_pad) and b lies inside its padded positions, in a row whose real tokens
-// fit its padded blocks. Uniform over the workgroup (scalar loads of the image).
+// padded count within n_pad) and b lies inside its padded positions, in a row that passes row_ok.
+// Uniform over the workgroup (scalar loads of the image).
 __device__ __forceinline__ bool block_live(const Rows& rows, int b, int n_tokens, int n_pad) {
   const int n = rows.n;
   if (n < 1 || n > kMaxRows || rows.start[n] != n_tokens || rows.pstart[n] > n_pad ||
       b * kBlk >= rows.pstart[n])
     return false;
   const int r = row_of_block(rows, b);
-  const int len = rows.start[r + 1] - rows.start[r];
-  return len >= 0 && rows.start[r] >= 0 && len <= rows.pstart[r + 1] - rows.pstart[r] &&
-         rows.pstart[r] % kBlk == 0 && rows.start[r + 1] <= n_tokens;
+  return row_ok(b, rows.start[r], rows.start[r + 1], rows.pstart[r], rows.pstart[r + 1],
+                rows.pstart[n], n_tokens);
 }
 
 // Where padded block b lies: its row r, the row's first real token, real length and first padded
@@ -116,7 +127,7 @@ __device__ __forceinline__ Where locate(const Rows& rows, int b, int n_tokens, i
   const int s0 = __builtin_amdgcn_readlane(stv, r), s1 = __builtin_amdgcn_readlane(stv, r + 1);
   const int p0 = __builtin_amdgcn_readlane(psv, r), p1 = __builtin_amdgcn_readlane(psv, r + 1);
   w.len = s1 - s0;
-  w.live = w.len >= 0 && s0 >= 0 && w.len <= p1 - p0 && p0 % kBlk == 0 && s1 <= n_tokens;
+  w.live = row_ok(b, s0, s1, p0, p1, pend, n_tokens);
   w.r = r;
   w.start = s0;
   w.pstart = p0;

@@ -374,3 +374,57 @@ def test_forward_forms_match_fp32(dev, lengths, heads):
     # the gradients' roundings are of the same kind (P, dS, the result): 5e-4 of the norm measured
     for got, want in zip((q.grad, k.grad, v.grad), grads):
         assert float((got.float() - want).norm() / want.norm()) <= 2e-3
+
+
+# Images no cm_attn_rows_image writes: (start, pstart, padded capacity, tokens still computed). A row
+# whose padded positions end past the image's, with an odd number of blocks inside it, for launches of
+# 64 (few blocks) and 128 queries per workgroup; a row that starts after the blocks attributed to it.
+BAD_IMAGES = {
+    "row_past_end_small": ([0, 100, 200], [0, 256, 192], 192, 0),
+    "row_past_end_large": ([0, 4200, 4300], [0, 4224, 4160], 4160, 0),
+    "row_after_block": ([0, 64, 128, 192], [0, 256, 64, 320], 320, 64),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", BAD_IMAGES)
+def test_inconsistent_rows_write_nothing(dev, name):
+    """Rows inconsistent with the launch are left alone by the forward and the backward: nothing is
+    written for them, and nothing outside the outputs."""
+    banner(f"inconsistent rows image {name}")
+    from claudemaxing_amd import _lib
+    from claudemaxing_amd.attention import _workspace
+
+    start, pstart, n_pad, done = BAD_IMAGES[name]
+    n, heads, groups = start[-1], 12, 2
+    words = torch.zeros(2 * 129 + 1, dtype=torch.int32)
+    words[:len(start)] = torch.tensor(start)
+    words[129:129 + len(pstart)] = torch.tensor(pstart)
+    words[258] = len(start) - 1
+    image = words.to(dev)
+    guard = 512 * 1536  # elements before and after each output, more than a misplaced block reaches
+
+    def guarded(numel, dtype, value):
+        buf = torch.full((numel + 2 * guard,), value, dtype=dtype, device=dev)
+        return buf, buf[guard:guard + numel]
+
+    q, k, v, do = (t.detach() for t in _inputs(dev, n, 3))
+    out_buf, out = guarded(n * heads * 128, torch.float16, 7.0)
+    lse_buf, lse = guarded(heads * n_pad, torch.float32, 7.0)
+    operands = [a for t in (q, k, v) for a in (t.data_ptr(), _lib.F16, t.stride(1), t.stride(2))]
+    ws = _workspace(n_pad, heads, groups, 128, False, dev)
+    stream = _lib.stream(dev)
+    _lib.call("cm_attn_fwd", *operands, image.data_ptr(), n, n_pad, heads, groups, 128, 0.088,
+              out.data_ptr(), lse.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+    ws = _workspace(n_pad, heads, groups, 128, True, dev)
+    grads = [guarded(n * h * 128, torch.float16, 7.0) for h in (heads, groups, groups)]
+    _lib.call("cm_attn_bwd", *operands, out.data_ptr(), do.data_ptr(), lse.data_ptr(),
+              image.data_ptr(), n, n_pad, heads, groups, 128, 0.088, grads[0][1].data_ptr(), _lib.F16,
+              grads[1][1].data_ptr(), grads[2][1].data_ptr(), _lib.F16, 1, ws.data_ptr(), ws.numel(),
+              stream)
+    torch.cuda.synchronize()
+    for buf, inner in [(out_buf, out), (lse_buf, lse), *grads]:
+        assert bool((buf[:guard] == 7).all()) and bool((buf[-guard:] == 7).all())
+        if inner is not lse:  # token-major: the tokens of rows that were left alone
+            assert bool((inner.view(n, -1)[done:] == 7).all())
+            assert done == 0 or not bool((inner.view(n, -1)[:done] == 7).all())

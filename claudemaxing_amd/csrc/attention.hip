@@ -413,8 +413,13 @@ __global__ __launch_bounds__(256) void attn_relayout_kernel(Jobs jobs, const Row
 //  - SPLIT: block (b, h) is 64 queries of one row, query head h (key/value head h / hpg); pair p
 //    takes the row's 64-key blocks p, p + 2, ... up to the diagonal block qb.
 //  - whole: 128 queries (blocks b and b + 1 of the row, b even in it), and all four wavefronts take
-//    every key block together: half the tile loads per query, no merge at the end, and half the LDS,
-//    so that a CU holds two workgroups and one's softmax runs beside the other's MFMAs.
+//    every key block together: half the tile loads per query, no hand-over at the end, and half the
+//    LDS, so that a CU holds two workgroups and one's softmax runs beside the other's MFMAs.
+// Both keep the even and the odd key blocks' softmax apart and merge them at the end with the same
+// operations (written as fused ones, so that the compiler's choice of contraction cannot tell them
+// apart): the form follows the launch's capacity, the bits do not. The whole form's second set of sums
+// stays in registers (238, none spilled): against one chain over all keys, whose bits were its own,
+// 30.7 -> 32.4 us at 8 x 512 tokens, 12 heads, 102 -> 105 at 3000, 28 heads, 324 -> 315 at 8191.
 constexpr int kTile = kBlk * kCh;  // a tile of 64 positions
 
 template <bool SPLIT>
@@ -445,7 +450,6 @@ __global__ __launch_bounds__(kThreads, SPLIT ? 1 : 2) void attn_fwd_kernel(
   const bool q_ok = ql < len;
   // the last key block of the workgroup's queries
   const int jb_last = SPLIT ? qb : min(qb + 1, (len - 1) / kBlk);
-  const int n_it = (jb_last + kSets) / kSets;
 
   const _Float16* kbase = k16 + (static_cast<int64_t>(g) * n_pad + p0) * kD;
   const _Float16* vbase = v16 + (static_cast<int64_t>(g) * n_pad + p0) * kD;
@@ -464,18 +468,26 @@ __global__ __launch_bounds__(kThreads, SPLIT ? 1 : 2) void attn_fwd_kernel(
     for (int ds = 0; ds < kD / 16; ++ds)
       qf[ds] = q_ok ? load8(q, q_dtype, off + ds * 16 + hh * 8) : zero8();
   }
-  floatx16 o[kD / 32];
+  // reference max (log2 domain), sum and O of the even and of the odd key blocks; the split form's
+  // wavefronts hold those of their own set
+  constexpr int kChains = SPLIT ? 1 : 2;
+  floatx16 o[kChains][kD / 32];
+  float m[kChains], l[kChains];
 #pragma unroll
-  for (int i = 0; i < kD / 32; ++i) o[i] = zero16();
-  float m = -__builtin_huge_valf(), l = 0.0f;  // reference max (log2 domain) and sum
+  for (int c = 0; c < kChains; ++c) {
+#pragma unroll
+    for (int i = 0; i < kD / 32; ++i) o[c][i] = zero16();
+    m[c] = -__builtin_huge_valf();
+    l[c] = 0.0f;
+  }
 
-  for (int it = 0; it < n_it; ++it) {
-    const int jb = kSets * it + set, st = it & 1;
+  // One key block, into the chain (o, m, l).
+  auto step = [&](int jb, int st, floatx16 (&o)[kD / 32], float& m, float& l) {
     cm::gemm::wait_vmcnt<0>();
     cm::gemm::lds_barrier();
     if (jb + kSets <= jb_last) issue(jb + kSets, st ^ 1);
     // set 1's last iteration when qb is even; keys that all follow this wavefront's queries
-    if (jb > jb_last || jb * kBlk > q0 + 31) continue;
+    if (jb > jb_last || jb * kBlk > q0 + 31) return;
     const uint4* kt = lds[set][st];
     const uint4* vt = kt + kTile;
     floatx16 s[2];
@@ -535,33 +547,45 @@ __global__ __launch_bounds__(kThreads, SPLIT ? 1 : 2) void attn_fwd_kernel(
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks)
         o[dt] = mfma(frag_t(vt, dt * 32, ks, lane), pf[ks], o[dt]);
+  };
+  if constexpr (SPLIT) {
+    const int n_it = (jb_last + 2) / 2;
+    for (int it = 0; it < n_it; ++it) step(2 * it + set, it & 1, o[0], m[0], l[0]);
+  } else {
+    for (int jb = 0; jb <= jb_last; jb += 2) {
+      step(jb, 0, o[0], m[0], l[0]);
+      if (jb < jb_last) step(jb + 1, 1, o[kChains - 1], m[kChains - 1], l[kChains - 1]);
+    }
   }
 
+  // the odd blocks' chain: in registers, or handed over by set 1 through its LDS region
   float* xf = nullptr;
-  float mt = m, a0 = 1.0f, a1 = 0.0f;
+  float m1, l1;
   if constexpr (SPLIT) {
-    // set 1 hands (o, m, l) of its blocks to set 0 through its LDS region
     cm::gemm::lds_barrier();
     xf = reinterpret_cast<float*>(lds[kSets - 1][0]) + wq * 66 * cm::kWave + lane;
     if (set == 1) {
 #pragma unroll
-      for (int i = 0; i < kD / 2; ++i) xf[i * cm::kWave] = o[i / 16][i % 16];
-      xf[64 * cm::kWave] = m;
-      xf[65 * cm::kWave] = l;
+      for (int i = 0; i < kD / 2; ++i) xf[i * cm::kWave] = o[0][i / 16][i % 16];
+      xf[64 * cm::kWave] = m[0];
+      xf[65 * cm::kWave] = l[0];
     }
     cm::gemm::lds_barrier();
     if (set == 1) return;
-    const float m1 = xf[64 * cm::kWave], l1 = xf[65 * cm::kWave];
-    mt = fmaxf(m, m1);
-    a0 = exp2_raw(m - mt);
-    a1 = exp2_raw(m1 - mt);  // 0 when set 1 had none
-    l = l * a0 + l1 * a1;
+    m1 = xf[64 * cm::kWave];
+    l1 = xf[65 * cm::kWave];
+  } else {
+    m1 = m[kChains - 1];
+    l1 = l[kChains - 1];
   }
+  const float mt = fmaxf(m[0], m1);
+  const float a0 = exp2_raw(m[0] - mt), a1 = exp2_raw(m1 - mt);  // a1 = 0 without odd blocks
+  const float lt = __builtin_fmaf(l[0], a0, l1 * a1);
   // positions past the row's padded blocks are another row's
   if (!SPLIT && q0 >= (len + kBlk - 1) / kBlk * kBlk) return;
-  if (hh == 0) lse2[static_cast<int64_t>(h) * n_pad + p0 + ql] = mt + __log2f(l);
+  if (hh == 0) lse2[static_cast<int64_t>(h) * n_pad + p0 + ql] = mt + __log2f(lt);
   if (!q_ok) return;
-  const float inv = 1.0f / l;
+  const float inv = 1.0f / lt;
   _Float16* orow = out + (static_cast<int64_t>(where.start + ql) * H + h) * kD;
 #pragma unroll
   for (int dt = 0; dt < kD / 32; ++dt)
@@ -572,9 +596,8 @@ __global__ __launch_bounds__(kThreads, SPLIT ? 1 : 2) void attn_fwd_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int e = g4 * 4 + i;
-        float ov = o[dt][e];
-        if constexpr (SPLIT) ov = ov * a0 + xf[(dt * 16 + e) * cm::kWave] * a1;
-        v[i] = static_cast<_Float16>(ov * inv);
+        const float odd = SPLIT ? xf[(dt * 16 + e) * cm::kWave] : o[kChains - 1][dt][e];
+        v[i] = static_cast<_Float16>(__builtin_fmaf(o[0][dt][e], a0, odd * a1) * inv);
       }
       *reinterpret_cast<h4*>(orow + dt * 32 + g4 * 8 + hh * 4) = v;
     }
@@ -998,11 +1021,12 @@ struct Workspace {
 };
 
 // The forward's form, by the launch's 64-query blocks times heads (the rows' lengths are only on the
-// device). The split form has one workgroup per block and the shorter serial chain, the whole form
-// half as many workgroups, two to a CU. Split / whole, forward with its relayout, us: 252 (4 rows of
-// 154-482 tokens, 12 heads) 19.8 / 22.1; 588 (2048 + 1000) 52 / 58; 672 (1500, 28 heads) 53 / 50;
-// 768 (8 x 512) 43 / 36; 960 (16 x 300) 44 / 36; 1316 (3000, 28 heads) 146 / 118; 1536 (8191) 355 /
-// 345. The one loss above the line is 1008 (2 x 2000, 16 heads): 84 / 86.
+// device; both forms give the same bits). The split form has one workgroup per block and the shorter
+// serial chain, the whole form half as many workgroups, two to a CU. Split / whole, forward with its
+// relayout in a graph, us: 264 (4 rows of 154-482 tokens, 12 heads) 16.4 / 21.2; 576 (2048 + 1000)
+// 48.1 / 61.4; 672 (1500, 28 heads) 49.1 / 51.0; 768 (8 x 512) 37.7 / 32.4; 960 (16 x 300) 38.0 / 31.3;
+// 1316 (3000, 28 heads) 128 / 106; 1536 (8191) 329 / 315; 3584 (8191, 28 heads) 757 / 603, (16 x 512, 28
+// heads) 122 / 77. The one loss above the line is 1024 (2 x 2000, 16 heads): 75.0 / 77.2.
 constexpr int64_t kSplitBelow = 768;
 
 // k16 and v16, and q16 (the rotated q of a fused RoPE)
@@ -1103,7 +1127,8 @@ int fwd_impl(const void* q, int q_dtype, int64_t sq_h, int64_t sq_t, const void*
                      s, jobs, rows, nt, np);
   if (int st = cm::launch_status()) return st;
   const void* qa = fused ? static_cast<const void*>(q16) : q;
-  const auto kernel = static_cast<int64_t>(H) * n_blocks < kSplitBelow ? attn_fwd_kernel<true> : attn_fwd_kernel<false>;
+  const bool split = static_cast<int64_t>(H) * n_blocks < kSplitBelow;
+  const auto kernel = split ? attn_fwd_kernel<true> : attn_fwd_kernel<false>;
   hipLaunchKernelGGL(kernel, dim3(H, n_blocks), dim3(kThreads), 0, s, qa,
                      fused ? CM_F16 : q_dtype, fused ? static_cast<int64_t>(n_pad) * kD : sq_h,
                      fused ? static_cast<int64_t>(kD) : sq_t, k16, v16, rows, nt, np, H / G, H,

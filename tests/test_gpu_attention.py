@@ -428,3 +428,22 @@ def test_inconsistent_rows_write_nothing(dev, name):
         if inner is not lse:  # token-major: the tokens of rows that were left alone
             assert bool((inner.view(n, -1)[done:] == 7).all())
             assert done == 0 or not bool((inner.view(n, -1)[:done] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths", [[154, 284, 482, 356], [1, 63, 64, 65, 128, 129, 192, 193, 700]],
+                         ids=["config5", "edges"])
+def test_capacity_leaves_the_bits(dev, lengths):
+    """One batch under its own padded count and under a capacity that puts the forward on 128 queries
+    per workgroup: the same bits, both ways."""
+    banner(f"attention capacity {lengths}")
+    from claudemaxing_amd.attention import PackedRows, packed_causal_attention
+
+    results = []
+    for capacity in (None, 4096):  # 4096 / 64 blocks x 12 heads = 768
+        q, k, v, do = _inputs(dev, sum(lengths), 6)
+        out = packed_causal_attention(q, k, v, PackedRows(_bounds(lengths), capacity))
+        out.backward(do)
+        results.append((out, q.grad, k.grad, v.grad))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

@@ -272,6 +272,17 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The same without a wait for the wavefront's own LDS reads, for a loop whose buffers are refilled no
+// earlier than two barriers after their last read (by then the arithmetic that uses the values has
+// waited for them). The compiler moves no memory access across it; the fences emit nothing.
+__device__ __forceinline__ void lds_barrier_reads_pending() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "singlethread");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "singlethread");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // Accumulators starting at zero, for epilogues with nothing to add to the product.
 struct ZeroStart {
   template <int TM, int TN>
@@ -589,9 +600,7 @@ __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int
     // the loads of stages kt + 1 .. kt + D - 1 may still be in flight when all were issued
     if (D > 1 && kt + D - 1 < n_kt) wait_vmcnt<(D - 1) * kDma>();
     else wait_vmcnt<0>();
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier_reads_pending();
     const uint4* st = lds + (kt % S) * kStage;
     constexpr int kStep = NM > NR ? NM : NR;  // slots per substep
     // substep s's slots multiply it and read substep s - 1 of the new stage

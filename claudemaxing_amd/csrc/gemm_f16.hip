@@ -13,6 +13,7 @@
 // of the three weights (~5 us alone, less among a layer's others) not counted: 65 tokens 8.8 / 12.8
 // against 28 / 21; 1276 15.1 / 15 against 30 / 35; 8192 52 / 56 against 90 / 115.
 #include "gemm_lds.h"
+#include "nf4_tiles.h"
 
 namespace {
 
@@ -92,23 +93,26 @@ struct EpiHalf {
   }
 };
 
-// SMALL: gemm_lds_small on SA ring stages
-template <int BM_, int BN_, int WM_, int WN_, int SA_, int SB_, int OCC_, bool SMALL_>
+// SMALL: gemm_lds_small on SA ring stages; SLICED: with its sums in slices
+template <int BM_, int BN_, int WM_, int WN_, int SA_, int SB_, int OCC_, bool SMALL_,
+          bool SLICED_ = false>
 struct Cfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, SA = SA_, SB = SB_, kOcc = OCC_;
-  static constexpr bool kSmall = SMALL_;
+  static constexpr bool kSmall = SMALL_, kSliced = SLICED_;
   static constexpr int kThreads = WM * WN * cm::kWave;
   static constexpr int kLds = (SA * BM + SB * BN) * 8;
   static_assert(kLds * 16 >= BM * (BN + 8) * 2, "the epilogue's tile fits the operands' rings");
 };
-using Narrow = Cfg<128, 64, 2, 2, 4, 4, 1, true>;
-using Small = Cfg<128, 128, 2, 2, 4, 4, 1, true>;
+template <bool SLICED>
+using Narrow = Cfg<128, 64, 2, 2, 4, 4, 1, true, SLICED>;
+template <bool SLICED>
+using Small = Cfg<128, 128, 2, 2, 4, 4, 1, true, SLICED>;
 using Large = Cfg<256, 256, 2, 4, 3, 2, 2, false>;
 
 template <class C, class SrcA, class SrcB>
 __global__ __launch_bounds__(C::kThreads, C::kOcc) void linear_f16_kernel(SrcA a, SrcB b, Outputs out,
                                                                           int M, int N, int K,
-                                                                          int remap) {
+                                                                          int remap, int slices) {
   __shared__ uint4 lds[C::kLds];
   int tm, tn;
   cm::gemm::tile_of(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x),
@@ -116,7 +120,8 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void linear_f16_kernel(SrcA a
   using Epi = EpiHalf<C::BM, C::BN, C::WM, C::WN>;
   Epi epi{out, M, N, tm * C::BM, tn * C::BN};
   if constexpr (C::kSmall) {
-    cm::gemm::gemm_lds_small<C::BM, C::BN, C::WM, C::WN, C::SA>(a, b, 0, K, tm, tn, epi, lds);
+    cm::gemm::gemm_lds_small<C::BM, C::BN, C::WM, C::WN, C::SA, C::kSliced>(
+        a, b, 0, K, tm, tn, epi, lds, slices);
   } else {
     cm::gemm::gemm_lds<C::BM, C::BN, C::WM, C::WN, C::SA, C::SB, SrcA, SrcB, Epi, cm::gemm::PlainA,
                        cm::gemm::kEdgeNever>(a, b, 0, K, tm, tn, epi, lds);
@@ -124,11 +129,12 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void linear_f16_kernel(SrcA a
 }
 
 template <class C, class SrcA, class SrcB>
-int launch(const SrcA& a, const SrcB& b, const Outputs& out, int M, int N, int K, hipStream_t s) {
+int launch(const SrcA& a, const SrcB& b, const Outputs& out, int M, int N, int K, int slices,
+           hipStream_t s) {
   const int64_t tiles = static_cast<int64_t>((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
   CM_CHECK_ARG(tiles <= 0x7fffffff);
   hipLaunchKernelGGL((linear_f16_kernel<C, SrcA, SrcB>), dim3(static_cast<unsigned>(tiles)),
-                     dim3(C::kThreads), 0, s, a, b, out, M, N, K, tiles % 8 == 0 ? 1 : 0);
+                     dim3(C::kThreads), 0, s, a, b, out, M, N, K, tiles % 8 == 0 ? 1 : 0, slices);
   return cm::launch_status();
 }
 
@@ -141,13 +147,26 @@ int64_t rounds(int64_t M, int64_t N, int64_t bm, int64_t bn) {
   return ((M + bm - 1) / bm * ((N + bn - 1) / bn) + 255) / 256;
 }
 
-template <class SrcA, class SrcB>
-int launch_best(const SrcA& a, const SrcB& b, const Outputs& out, int M, int N, int K,
+template <bool SLICED, class SrcA, class SrcB>
+int launch_best(const SrcA& a, const SrcB& b, const Outputs& out, int M, int N, int K, int slices,
                 hipStream_t s) {
-  if (rounds(M, N, 128, 64) <= 1) return launch<Narrow>(a, b, out, M, N, K, s);
-  if (rounds(M, N, 256, 256) * 3 <= rounds(M, N, 128, 128))
-    return launch<Large>(a, b, out, M, N, K, s);
-  return launch<Small>(a, b, out, M, N, K, s);
+  if (rounds(M, N, 128, 64) <= 1) return launch<Narrow<SLICED>>(a, b, out, M, N, K, slices, s);
+  // 256 x 256 tiles sum in one slice (their accumulators leave no registers for a second set); more
+  // than 512 tiles of 128 x 128, which they need, are never split
+  if constexpr (!SLICED) {
+    if (rounds(M, N, 256, 256) * 3 <= rounds(M, N, 128, 128))
+      return launch<Large>(a, b, out, M, N, K, slices, s);
+  }
+  return launch<Small<SLICED>>(a, b, out, M, N, K, slices, s);
+}
+
+// Slices in which the input gradient of M rows is summed over its contraction of `stages` 64-column
+// stages: those the NF4-fused GEMM splits it into (nf4_tiles.h), so that the gradient has that kernel's
+// bits. Summed in one chain, q/k/v's at 1276 tokens is 8e-6 of its norm away, as close to the exact one
+// (4.7e-4), and the training step's adapter gradients, 28 layers further, 4e-3. The slices' second set
+// of accumulators costs 15.7 -> 16.4 us at 1276 tokens of 1536 -> 1536 + 256 + 256, 12.5 -> 14.0 at 65.
+int dx_slices(int M, int K, int stages) {
+  return K % 128 ? 1 : cm::nf4_tiles(M, K, K % 256 == 0, true, stages).split;
 }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -178,7 +197,7 @@ extern "C" int cm_linear_f16_fwd(const void* x, int64_t ldx, int64_t M, int K, c
   const RowMajor a{static_cast<const _Float16*>(x), ldx, m, K};
   const RowMajor b{static_cast<const _Float16*>(w), K, n, K};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return launch_best(a, b, o, m, n, K, s);
+  return launch_best<false>(a, b, o, m, n, K, 1, s);
 }
 
 extern "C" int cm_linear_f16_bwd(const void* const* grad, const int64_t* ldg, int64_t M, int n_in,
@@ -210,5 +229,7 @@ extern "C" int cm_linear_f16_bwd(const void* const* grad, const int64_t* ldg, in
   o.ld[0] = ldx;
   o.first[1] = o.first[2] = 0x7fffffff;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return launch_best(g, b, o, m, K, n, s);
+  const int slices = dx_slices(m, K, n / 64);
+  return slices > 1 ? launch_best<true>(g, b, o, m, K, n, slices, s)
+                    : launch_best<false>(g, b, o, m, K, n, 1, s);
 }

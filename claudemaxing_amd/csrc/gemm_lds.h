@@ -540,10 +540,13 @@ __device__ __forceinline__ void gemm_lds(const SrcA& A, const SrcB& B, int k_beg
 // multiplied substep by substep, the registers of each finished substep are refilled from stage kt.
 // A fragment then has three substeps of MFMAs to arrive in. One ring of S stages of both operands,
 // loaded S - 2 stages ahead: the slot that stage kt's loads fill was last read two barriers ago, so
-// the barrier waits for no fragment read.
-template <int BM, int BN, int WM, int WN, int S, class SrcA, class SrcB, class Epi>
+// the barrier waits for no fragment read. With SLICED the n_kt stages are summed in `slices` parts of
+// their own, stages [s n_kt / slices, (s + 1) n_kt / slices), added in order: the sums of a contraction
+// split over workgroups. Slices have at least D + 3 stages.
+template <int BM, int BN, int WM, int WN, int S, bool SLICED, class SrcA, class SrcB, class Epi>
 __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int k_begin, int k_end,
-                                               int tm, int tn, Epi& epi, uint4* lds) {
+                                               int tm, int tn, Epi& epi, uint4* lds,
+                                               int slices = 1) {
   constexpr int BK = 64, NW = WM * WN, KS = BK / 16, D = S - 2;
   constexpr int WTM = BM / WM, WTN = BN / WN, TM = WTM / 32, TN = WTN / 32;
   static_assert(TM * 32 == WTM && TN * 32 == WTN, "wave tiles are multiples of 32");
@@ -584,9 +587,11 @@ __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int
       bf[ks][r - TM] = LB::frag(st + kTileA, brow + (r - TM) * 32, ch);
     }
   };
-  auto mfma = [&](int ks, int g) {
+  // fresh: the sum starts anew with substep 0
+  auto mfma = [&](int ks, int g, auto fresh) {
     const int i = g / TN, j = g % TN;
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks][i], bf[ks][j], acc[i][j], 0, 0, 0);
+    const floatx16 c = decltype(fresh)::value && ks == 0 ? floatx16{} : acc[i][j];
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks][i], bf[ks][j], c, 0, 0, 0);
   };
   static_for<D>([&](auto sc) {
     constexpr int s = decltype(sc)::value;
@@ -596,7 +601,7 @@ __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int
     }
   });
   epi.template started<TM, TN>(acc);
-  auto stage = [&](int kt, auto first, auto loads) {
+  auto stage = [&](int kt, auto first, auto loads, auto fresh) {
     // the loads of stages kt + 1 .. kt + D - 1 may still be in flight when all were issued
     if (D > 1 && kt + D - 1 < n_kt) wait_vmcnt<(D - 1) * kDma>();
     else wait_vmcnt<0>();
@@ -606,7 +611,7 @@ __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int
     // substep s's slots multiply it and read substep s - 1 of the new stage
     static_for<(KS + 1) * kStep>([&](auto sc) {
       constexpr int slot = decltype(sc)::value, ks = slot / kStep, m = slot % kStep;
-      if constexpr (ks < KS && m < NM && !decltype(first)::value) mfma(ks, m);
+      if constexpr (ks < KS && m < NM && !decltype(first)::value) mfma(ks, m, fresh);
       if constexpr (ks > 0 && m < NR) read(st, ks - 1, m);
       if constexpr (decltype(loads)::value) {
         static_for<kDma>([&](auto qc) {
@@ -617,16 +622,45 @@ __device__ __forceinline__ void gemm_lds_small(const SrcA& A, const SrcB& B, int
       __builtin_amdgcn_sched_barrier(0);
     });
   };
+  floatx16 sum[SLICED ? TM : 1][SLICED ? TN : 1];  // of the finished slices
+  if constexpr (SLICED) ZeroStart::start<TM, TN>(sum, 0, 0, 0);
   if (n_kt > 0) {
-    if (D < n_kt) stage(0, std::true_type{}, std::true_type{});
-    else stage(0, std::true_type{}, std::false_type{});
+    constexpr auto kYes = std::true_type{};
+    constexpr auto kNo = std::false_type{};
+    if (D < n_kt) stage(0, kYes, kYes, kNo);
+    else stage(0, kYes, kNo, kNo);
+    int slice = 1, slice_at = SLICED && slices > 1 ? n_kt / slices : n_kt;
     int kt = 1;
-    for (; kt + D < n_kt; ++kt) stage(kt, std::false_type{}, std::true_type{});
-    for (; kt < n_kt; ++kt) stage(kt, std::false_type{}, std::false_type{});
+    for (; kt + D < n_kt; ++kt) {
+      stage(kt, kNo, kYes, kNo);
+      if constexpr (SLICED) {
+        if (kt != slice_at) continue;
+        // the slice's last stage, kt - 1, is multiplied; the next stage's slots start a new one
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sum[i][j][r] += acc[i][j][r];
+        ++slice;
+        slice_at = slice < slices ? slice * n_kt / slices : n_kt;
+        ++kt;
+        stage(kt, kNo, kYes, kYes);
+      }
+    }
+    for (; kt < n_kt; ++kt) stage(kt, kNo, kNo, kNo);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int g = 0; g < NM; ++g) mfma(ks, g);
+      for (int g = 0; g < NM; ++g) mfma(ks, g, kNo);
+  }
+  if constexpr (SLICED) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += sum[i][j][r];
   }
   epi.template apply<TM, TN>(acc, m0 + wm * WTM, n0 + wn * WTN, lane, lds);
 }

@@ -36,6 +36,7 @@
 
 #include "common.h"
 #include "gemm_lds.h"
+#include "nf4_tiles.h"
 
 namespace {
 
@@ -472,7 +473,6 @@ constexpr int kConsumers = 8;  // MFMA wavefronts: 4 x 2 (256-row tiles) or 2 x 
 constexpr int kProducers = 4;
 constexpr int kWsThreads = (kConsumers + kProducers) * 64;
 constexpr int kRing = 3;
-constexpr int kWsBN = 128;
 
 // One global_load_lds_dword: lane l's 4 bytes from g land at lds_lane0 + 4 l (wave-uniform base in
 // M0); issued like gemm::dma16.
@@ -875,7 +875,7 @@ int log2_exact(int64_t v) {
   return s;
 }
 
-constexpr int kCUs = 256;
+constexpr int kCUs = cm::kNf4CUs;
 
 template <int BM, int BN, bool TRANS>
 int launch_cfg(const Args& a, int n_tiles, hipStream_t stream) {
@@ -954,7 +954,6 @@ struct Plan {
 
 Plan plan_for(const Args& a, bool trans) {
   Plan p{};
-  const int64_t tb = (static_cast<int64_t>(a.m) + kWsBN - 1) / kWsBN;
   int64_t rows_total = 0;
   bool all128 = true, all256 = true;
   for (int i = 0; i < a.n_w; ++i) {
@@ -971,40 +970,13 @@ Plan plan_for(const Args& a, bool trans) {
   const bool e256 = trans ? a.cols % 256 == 0 : all256;
   p.n_out = trans ? a.cols : (a.n_w == 1 ? a.w[0].rows : 0);
   if (e128) {
+    const cm::Nf4Tiles t = cm::nf4_tiles(a.m, extent, e256, trans || a.n_w == 1,
+                                         trans ? a.n_stages : a.cols / kBK);
     p.ws = true;
-    p.bn = kWsBN;
-    p.bm = e256 ? 256 : 128;
-    p.tiles = extent / p.bm * tb;
-    if (p.bm == 256 && p.tiles < kCUs / 2) {
-      p.bm = 128;
-      p.tiles = extent / p.bm * tb;
-    }
-    // 256-token tiles expand each weight element half as often; taken when they, split over the
-    // contraction where that is allowed, still give most CUs a workgroup
-    const int64_t tb2 = (static_cast<int64_t>(a.m) + 255) / 256;
-    const int64_t tiles2 = extent / 128 * tb2;
-    const bool can_split = trans || a.n_w == 1;
-    const int n_stages_all = trans ? a.n_stages : a.cols / kBK;
-    int64_t sp2 = 1;
-    if (can_split && tiles2 < kCUs * 3 / 4) {
-      sp2 = kCUs / (tiles2 > 0 ? tiles2 : 1);
-      if (sp2 > 8) sp2 = 8;
-      if (sp2 > n_stages_all / 8) sp2 = n_stages_all / 8;
-      if (sp2 < 1) sp2 = 1;
-    }
-    if (a.m >= 384 && tiles2 * sp2 >= kCUs * 3 / 4) {
-      p.bm = 128;
-      p.bn = 256;
-      p.tiles = tiles2;
-    }
-    const int n_all = trans ? a.n_stages : a.cols / kBK;
-    p.split = 1;
-    if (p.tiles < 3 * kCUs / 4 && (trans || a.n_w == 1)) {
-      int64_t sp = kCUs / (p.tiles > 0 ? p.tiles : 1);
-      if (sp > 8) sp = 8;
-      if (sp > n_all / 8) sp = n_all / 8;
-      if (sp > 1) p.split = static_cast<int>(sp);
-    }
+    p.bm = t.bm;
+    p.bn = t.bn;
+    p.tiles = t.tiles;
+    p.split = t.split;
     p.ws_bytes = p.split > 1 ? int64_t{4} * p.split * a.m * p.n_out : 0;
     return p;
   }

@@ -58,6 +58,39 @@ def test_linear_rows(dev, m, k, sizes):
     assert bool(((dx.double() - ref).abs() <= _bound(merged, w, ref)).all())
 
 
+# q, k, v weights as NF4, and token counts on both sides of where the fused GEMM's tiles and the number
+# of slices of its input gradient change (8 to 1 slices: 4 at 1276 tokens of the first)
+NF4_SHAPES = [(m, 1536, (1536, 256, 256)) for m in (1, 65, 257, 640, 1276, 2049, 2500, 3400, 5400)]
+NF4_SHAPES += [(300, 2048, (2048, 256, 256)), (1276, 2048, (2048, 256, 256)),
+               (900, 256, (1088, 64, 64)), (1276, 384, (640, 192, 64)), (700, 192, (192, 64, 64))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,sizes", NF4_SHAPES)
+def test_linear_rows_has_the_fused_gemms_bits(dev, m, k, sizes):
+    """Both ways, on expanded weights, the bits of the GEMM that expands them inside: the same fp16
+    operands, the sums in the same order (the input gradient's in the same slices)."""
+    from claudemaxing_amd.nf4 import quantize_nf4
+    from claudemaxing_amd.nf4_linear import (expand_rows, linear_rows_bwd, linear_rows_fwd,
+                                             nf4_linear_bwd, nf4_linear_fwd)
+
+    g = torch.Generator(device=dev).manual_seed(m + k)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device=dev)
+
+    pairs = []
+    for s in sizes:
+        packed, state = quantize_nf4((normal(s, k) * 0.02).cpu(), 64, True)
+        pairs.append((packed.to(dev), state.to(dev)))
+    x, grads = normal(m, k).half(), [normal(m, s).half() for s in sizes]
+    w = expand_rows(pairs)
+    biases = [normal(s).half() for s in sizes]
+    for a, b in zip(linear_rows_fwd(x, w, list(sizes), biases), nf4_linear_fwd(x, pairs, biases)):
+        assert torch.equal(a, b)
+    assert torch.equal(linear_rows_bwd(grads, w, list(sizes)), nf4_linear_bwd(grads, pairs))
+
+
 @pytest.mark.gpu
 def test_linear_f16_refuses(dev):
     from claudemaxing_amd import _lib

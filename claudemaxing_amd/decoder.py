@@ -71,8 +71,16 @@ def patch_qwen2_decoder_residual():
                              position_ids=position_ids, past_key_values=past_key_values,
                              use_cache=use_cache, position_embeddings=position_embeddings,
                              **kwargs)
-            n1, n2 = self.input_layernorm, self.post_attention_layernorm
             expand.expand_layer(self, hidden_states)  # the layer's NF4 expansions, one launch
+            try:
+                return fused(self, hidden_states, attention_mask, position_ids, past_key_values,
+                             use_cache, position_embeddings, kwargs)
+            finally:
+                expand.drop(hidden_states.device)
+
+        def fused(self, hidden_states, attention_mask, position_ids, past_key_values, use_cache,
+                  position_embeddings, kwargs):
+            n1, n2 = self.input_layernorm, self.post_attention_layernorm
             y, residual = norm_pass(hidden_states, n1.weight, n1.variance_epsilon)
             attn, _ = self.self_attn(hidden_states=y, attention_mask=attention_mask,
                                      position_ids=position_ids, past_key_values=past_key_values,
@@ -84,9 +92,7 @@ def patch_qwen2_decoder_residual():
             else:
                 h = residual + attn
                 y = n2(h)
-            out = self.mlp(y, residual=h) if _mlp_takes_residual(self.mlp) else h + self.mlp(y)
-            expand.drop(hidden_states.device)
-            return out
+            return self.mlp(y, residual=h) if _mlp_takes_residual(self.mlp) else h + self.mlp(y)
 
         return forward
 

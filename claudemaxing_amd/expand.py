@@ -7,14 +7,14 @@ the forward and again in the backward. Those are short launches (6-9 us each at
 Qwen2.5-1.5B's shapes, of which the ramp and the drain of a launch are a large part), so the
 layer issues them together, through cm_nf4_dequant_group:
 
-* forward: the patched decoder layer calls `expand_layer` first. It expands the weights whose
-  products will take the dequant route at this token count (o and down into their own fp16
-  weights, gate and up into one [2F, K] weight, the MLP's merged product, q, k and v one under
-  another where NF4QKV runs) in one launch and leaves them for `take` / `take_pair` / `take_rows`,
-  which the o and down projections' MatMulNF4, the MLP and NF4QKV call instead of expanding; the
-  layer calls `drop` at its end.
+* forward: the patched decoder layer calls `expand_layer` first and `drop` at its end, also when it
+  raises. In between, the first consumer that asks for an expansion (`take` / `take_pair` /
+  `take_rows`, called by the o and down projections' MatMulNF4, the MLP and NF4QKV instead of
+  expanding) sets off the group: its own weights and those of the layer's later products that will
+  take the dequant route at this token count (o and down into their own fp16 weights, gate and up
+  into one [2F, K] weight, the MLP's merged product; q, k and v one under another when NF4QKV asks).
 * backward: the down projection's input gradient is the first expansion of the layer's
-  backward. `backward_group`, called there, finds the layer's group (recorded by `expand_layer`)
+  backward. `backward_group`, called there, finds the layer's group (recorded in its forward)
   and expands down, gate/up, o and q/k/v together the same way, for the MLP's input gradient, then
   the o projection's and NF4QKV's.
 
@@ -22,136 +22,154 @@ Every weight is expanded by the dequant kernel's own code (the values of dequant
 for bit), and a consumer that finds nothing left for it expands its weight itself: the values
 and the routes are the same with or without the grouping. Everything runs on the caller's
 current stream, in order, so a captured step replays it as it runs eagerly.
+
+What is left belongs to one pass: it is handed out on the stream it was expanded on, inside the
+backward pass (autograd graph task) it was expanded in, or outside of any, and only for the very
+weights it was expanded from, unmodified since. So a backward that ends early (a partial
+torch.autograd.grad, an exception) leaves nothing that a later call, another stream or a graph
+capture could take; the next layer's pass on the device frees it.
 """
 
 import weakref
 
 import torch
 
-_READY = {}   # device index -> {key: fp16 weight}; key = packed pointer, ("pair", gate, up) or
-              # ("rows", q, k, v)
+from . import _lib
+from . import nf4_linear as _nl  # imports this module in turn: used by attribute only
+
+_READY = {}   # device index -> _Left: what the current layer's group left
 _GROUPS = {}  # down projection's packed pointer -> weak reference to its decoder layer
 
 
-def _nf4_module(m):
-    from .nf4_linear import NF4Linear
+def _version(t):
+    try:
+        return t._version
+    except (RuntimeError, AttributeError):  # an inference tensor has none; no tensor
+        return None
 
-    return (isinstance(m, NF4Linear) and m.compute_dtype == torch.float16
+
+def _sources(pairs):
+    return [(p, s, _version(p), _version(getattr(s, "absmax", None))) for p, s in pairs]
+
+
+class _Left(dict):
+    """The expansions one group launch left: {key: (fp16 weight, the weights it was expanded from and
+    their versions)} with key = packed pointer, ("pair", gate, up) or ("rows", q, k, v). The weights
+    are held, so no other can have their address. `pending`: the layer whose forward has not asked
+    for anything yet, with what its plan needs."""
+
+    def __init__(self, device, pending=None):
+        super().__init__()
+        self.device, self.pending = device, pending
+        self.task = torch._C._current_graph_task_id()  # -1 outside of a backward pass
+        self.stream = _lib.stream(device) if device.type == "cuda" else None
+
+    def leave(self, key, weight, pairs):
+        self[key] = weight, _sources(pairs)
+
+    def take(self, key, pairs):
+        if self.task != torch._C._current_graph_task_id() or (
+                self.stream is not None and self.stream != _lib.stream(self.device)):
+            return None
+        if self.pending is not None:
+            pending, self.pending = self.pending, None
+            _forward_group(self, pairs if key.__class__ is tuple and key[0] == "rows" else None,
+                           *pending)
+        weight, sources = self.pop(key, (None, ()))
+        for (packed, state), (p, s, version, scales) in zip(pairs, sources):
+            if (packed is not p or state is not s or _version(p) != version
+                    or _version(getattr(s, "absmax", None)) != scales):
+                return None
+        return weight
+
+
+def _take(device, key, pairs):
+    ready = _READY.get(device.index)
+    if ready is None:
+        return None
+    return ready.take(key, pairs) if isinstance(ready, _Left) else ready.pop(key, None)
+
+
+def _nf4_module(m):
+    return (isinstance(m, _nl.NF4Linear) and m.compute_dtype == torch.float16
             and not (m._forward_hooks or m._forward_pre_hooks))
 
 
 def _single_route(m, tokens):
     """MatMulNF4 expands this layer's weight with the dequant kernel (not the fused GEMM) for
     `tokens` rows in fp16."""
-    from .nf4_linear import fused_pays, fused_supported
-
     if not _nf4_module(m):
         return False
     state = m.quant_state
-    return not (fused_supported(m.packed, state) and fused_pays(tokens, *state.shape))
+    return not (_nl.fused_pays(tokens, *state.shape) and _nl.fused_supported(m.packed, state))
 
 
-def _pair_route(mlp, tokens, x_dtype):
+def _pair_route(gp, up, tokens, x_dtype):
     """The MLP's recompute takes its merged gate/up product for `tokens` rows of an x_dtype
     input (swiglu_recompute._merged_route), through MLPInputRecompute: a call with gradients
     enabled (the MLP input of a decoder layer with trainable adapters needs its gradient)."""
     from . import swiglu_recompute as SR
 
-    gp, up = getattr(mlp, "gate_proj", None), getattr(mlp, "up_proj", None)
-    if not (_nf4_module(gp) and _nf4_module(up)) or gp.bias is not None or up.bias is not None:
-        return False
-    if not (torch.is_grad_enabled() and SR._frozen(gp) and SR._frozen(up)):
-        return False
-    return SR._merged_route(tokens, gp.packed.is_cuda, x_dtype, gp, up)
-
-
-def _qkv_route(attn, hidden):
-    """The NF4Linear bases of q, k and v when this call's attention runs NF4QKV (its input, the
-    norm's output, has hidden's shape, dtype and device), else None."""
-    from . import qkv
-    from ._patching import tagged
-
-    if attn is None or not tagged(type(attn).forward, "fused_qkv") or attn._forward_pre_hooks:
-        return None
-    if not all(hasattr(attn, n) for n in ("q_proj", "k_proj", "v_proj")):
-        return None
-    if not qkv._fused_layout(attn, hidden):
-        return None
-    return attn.q_proj.base_layer, attn.k_proj, attn.v_proj.base_layer
+    return (_nf4_module(gp) and _nf4_module(up) and gp.bias is None and up.bias is None
+            and SR._frozen(gp) and SR._frozen(up)
+            and SR._merged_route(tokens, gp.packed.is_cuda, x_dtype, gp, up))
 
 
 def _rows_key(packed):
     return ("rows", *(p.data_ptr() for p in packed))
 
 
-def _issue(dev, singles, pair, rows):
-    """Expand `singles` (NF4Linear modules), `pair` ((gate, up) or None) and `rows` ((q, k, v) or
-    None) in one launch; the {key: weight} map of the results."""
-    from .nf4_linear import dequantize_group
-
-    pairs, outs, ready = [], [], {}
+def _issue(left, singles, pair, rows):
+    """Expand `singles` (NF4Linear modules), `pair` ((gate, up) or None) and `rows` (the (packed,
+    QuantState) of q, k and v or None) in one launch, into `left`."""
+    pairs, pointers = [], []
+    empty = dict(dtype=torch.float16, device=left.device)
     for m in singles:
-        w = torch.empty(m.quant_state.shape, dtype=torch.float16, device=dev)
+        w = torch.empty(m.quant_state.shape, **empty)
         pairs.append((m.packed, m.quant_state))
-        outs.append(w)
-        ready[m.packed.data_ptr()] = w
+        pointers.append(w.data_ptr())
+        left.leave(m.packed.data_ptr(), w, pairs[-1:])
     if pair is not None:
         gp, up = pair
         f, k = gp.quant_state.shape
-        w2 = torch.empty(2 * f, k, dtype=torch.float16, device=dev)
+        w2 = torch.empty(2 * f, k, **empty)
         pairs += [(gp.packed, gp.quant_state), (up.packed, up.quant_state)]
-        outs += [w2[:f], w2[f:]]
-        ready[("pair", gp.packed.data_ptr(), up.packed.data_ptr())] = w2
+        pointers += [w2.data_ptr(), w2.data_ptr() + 2 * f * k]
+        left.leave(("pair", gp.packed.data_ptr(), up.packed.data_ptr()), w2, pairs[-2:])
     if rows is not None:
-        sizes = [int(m.quant_state.shape[0]) for m in rows]
-        w3 = torch.empty(sum(sizes), int(rows[0].quant_state.shape[1]), dtype=torch.float16,
-                         device=dev)
-        pairs += [(m.packed, m.quant_state) for m in rows]
-        outs += w3.split(sizes)
-        ready[_rows_key([m.packed for m in rows])] = w3
-    dequantize_group(pairs, outs, checked=True)
-    return ready
+        k = int(rows[0][1].shape[1])
+        w3 = torch.empty(sum(int(state.shape[0]) for _, state in rows), k, **empty)
+        pairs += rows
+        at = w3.data_ptr()
+        for _, state in rows:
+            pointers.append(at)
+            at += 2 * int(state.shape[0]) * k
+        left.leave(_rows_key([packed for packed, _ in rows]), w3, rows)
+    _nl.expand_to(pairs, pointers, torch.float16, left.device)
 
 
-def _plan(layer, hidden, tokens):
-    """(singles, pair, rows, o, down, rows_bwd) of the layer for this call: the o / down modules whose
-    products take the dequant route, the (gate, up) pair of the merged product or None, the (q, k, v)
-    of NF4QKV or None, the o and down modules, and rows again when the backward multiplies by them
-    (the first layer's input needs no gradient). Kept on the layer per (token count, dtype, device,
-    gradient and autocast mode, training, modules): the routes depend on nothing else. The
-    backward's group reads the plan of the layer's last forward."""
+def _forward_group(left, rows, layer, tokens, x_dtype, grad, x_grad):
+    """The group of a layer's forward on `tokens` rows of an x_dtype input (grad: gradients enabled;
+    x_grad: the input needs one), set off by the first consumer (rows: NF4QKV's weights when it is
+    that): expanded when it has at least two weights, and recorded for the backward: (o and down
+    modules whose products take the dequant route, (gate, up) of the merged product or None, q/k/v
+    when the backward multiplies by them too). Found anew for each pass, by the questions the
+    consumers ask."""
     attn, mlp = getattr(layer, "self_attn", None), getattr(layer, "mlp", None)
-    o = getattr(attn, "o_proj", None)
-    down = getattr(mlp, "down_proj", None)
+    o, down = getattr(attn, "o_proj", None), getattr(mlp, "down_proj", None)
     gp, up = getattr(mlp, "gate_proj", None), getattr(mlp, "up_proj", None)
-    q, k, v = (getattr(attn, n, None) for n in ("q_proj", "k_proj", "v_proj"))
-    key = (tokens, hidden.dtype, hidden.device, torch.is_grad_enabled(),
-           torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"),
-           getattr(q, "training", None), getattr(v, "training", None), hidden.is_contiguous(),
-           hidden.requires_grad,
-           id(o), id(down), id(gp), id(up), id(q), id(k), id(v))
-    cached = layer.__dict__.get("_cm_expand_plan")
-    if cached is not None and cached[0] == key:
-        return cached[1]
-    singles = [m for m in (o, down) if _single_route(m, tokens)]
-    pair = (gp, up) if _pair_route(mlp, tokens, hidden.dtype) else None
-    rows = _qkv_route(attn, hidden)
-    plan = (singles, pair, rows, o, down, rows if hidden.requires_grad else None)
-    layer.__dict__["_cm_expand_plan"] = (key, plan)
-    return plan
-
-
-def expand_layer(layer, hidden):
-    """At the start of a decoder layer's forward on `hidden` (its input, [..., H] on the GPU):
-    expand, in one launch, the o / down projections' weights, the merged gate/up weight and the q/k/v
-    weights that this call's products will expand, when there are at least two."""
-    drop(hidden.device)
-    singles, pair, rows, o, down, _ = _plan(layer, hidden, hidden.numel() // max(hidden.shape[-1], 1))
+    o = o if _single_route(o, tokens) else None
+    down = down if _single_route(down, tokens) else None
+    pair = (gp, up) if grad and _pair_route(gp, up, tokens, x_dtype) else None
+    singles = [m for m in (o, down) if m is not None]
+    if grad:
+        layer.__dict__.pop("_cm_expand_plan", None)
     if len(singles) + (2 if pair else 0) + (3 if rows else 0) < 2:
         return
-    _READY[hidden.device.index] = _issue(hidden.device, singles, pair, rows)
-    if down in singles and torch.is_grad_enabled():
-        # the backward finds the layer (and its plan: the same routes) from the down weight
+    _issue(left, singles, pair, rows)
+    if down is not None and grad:
+        # the backward finds the layer (and its group: the same routes) from the down weight
+        layer.__dict__["_cm_expand_plan"] = (o, down, pair, rows if x_grad else None)
         ref = _GROUPS.get(down.packed.data_ptr())
         if ref is None or ref() is not layer:
             if len(_GROUPS) > 1024:  # entries of models that are gone
@@ -159,50 +177,52 @@ def expand_layer(layer, hidden):
             _GROUPS[down.packed.data_ptr()] = weakref.ref(layer)
 
 
-def take(packed, dtype):
-    """The fp16 expansion of `packed` left by the group launch, once; None when there is none
-    (or `dtype` is not fp16)."""
-    ready = _READY.get(packed.device.index)
-    if not ready or dtype != torch.float16:
+def expand_layer(layer, hidden):
+    """At the start of a decoder layer's forward on `hidden` (its input, [..., H] on the GPU): the
+    first expansion asked for until `drop` sets off the layer's group."""
+    _READY[hidden.device.index] = _Left(hidden.device, (
+        layer, hidden.numel() // max(hidden.shape[-1], 1), hidden.dtype, torch.is_grad_enabled(),
+        hidden.requires_grad))
+
+
+def take(packed, dtype, state=None):
+    """The fp16 expansion of `packed` (with its QuantState) left by the group launch, once; None when
+    there is none (or `dtype` is not fp16)."""
+    if dtype != torch.float16:
         return None
-    return ready.pop(packed.data_ptr(), None)
+    return _take(packed.device, packed.data_ptr(), [(packed, state)])
 
 
 def take_pair(gate_proj, up_proj):
     """The merged [2F, K] fp16 weight [Wg; Wu] left by the group launch, once; or None."""
-    ready = _READY.get(gate_proj.packed.device.index)
-    if not ready:
-        return None
-    return ready.pop(("pair", gate_proj.packed.data_ptr(), up_proj.packed.data_ptr()), None)
+    gate, up = gate_proj.packed, up_proj.packed
+    return _take(gate.device, ("pair", gate.data_ptr(), up.data_ptr()),
+                 [(p.packed, getattr(p, "quant_state", None)) for p in (gate_proj, up_proj)])
 
 
 def take_rows(pairs):
     """The stacked fp16 weights of `pairs` [(packed, QuantState)] left by the group launch, once; or
     None."""
-    ready = _READY.get(pairs[0][0].device.index)
-    if not ready:
-        return None
-    return ready.pop(_rows_key([p for p, _ in pairs]), None)
+    return _take(pairs[0][0].device, _rows_key([p for p, _ in pairs]), pairs)
 
 
 def backward_group(packed, dtype):
     """In the backward, for the down projection of a layer whose forward recorded a group: expand
-    down, the merged gate/up weight, o and q/k/v in one launch, leave the others for `take_pair` /
-    `take` / `take_rows`, and return the down weight; None for any other weight."""
+    down, the merged gate/up weight, o and q/k/v in one launch and leave them for `take`,
+    `take_pair` and `take_rows`; the down weight, or None for any other weight."""
     ref = _GROUPS.get(packed.data_ptr())
     layer = None if ref is None else ref()
     plan = None if layer is None else layer.__dict__.get("_cm_expand_plan")
     if plan is None or dtype != torch.float16:
         return None
-    singles, pair, _, o, down, rows = plan[1]
-    if down not in singles or down.packed is not packed:
+    o, down, pair, rows = plan
+    if down.packed is not packed:
         return None
-    singles = [down] + ([o] if o in singles else [])
     drop(packed.device)
-    ready = _issue(packed.device, singles, pair, rows)
-    w = ready.pop(packed.data_ptr())
-    _READY[packed.device.index] = ready
-    return w
+    left = _Left(packed.device)
+    _issue(left, [down] if o is None else [down, o], pair, rows)
+    _READY[packed.device.index] = left
+    return left[packed.data_ptr()][0]
 
 
 def drop(device):

@@ -164,10 +164,14 @@ def dequantize_group(pairs, outs, checked=False):
                 or out.numel() != int(state.shape[0]) * int(state.shape[1])):
             raise ValueError("dequantize_group: each output must be a contiguous tensor of its "
                              "weight's size, all of one dtype, on the weights' device")
-    w = _plain_weights(pairs)[0]
-    out_arr = (ctypes.c_void_p * len(outs))(*[o.data_ptr() for o in outs])
-    _lib.call("cm_nf4_dequant_group", w, len(pairs), out_arr, _lib.dtype_code(dtype),
-              _lib.stream(outs[0].device))
+    expand_to(pairs, [o.data_ptr() for o in outs], dtype, outs[0].device)
+
+
+def expand_to(pairs, pointers, dtype, device):
+    """dequantize_group to the addresses `pointers`, each with room for its weight in `dtype`."""
+    _lib.call("cm_nf4_dequant_group", _plain_weights(pairs)[0], len(pairs),
+              (ctypes.c_void_p * len(pairs))(*pointers), _lib.dtype_code(dtype),
+              _lib.stream(device))
 
 
 # Products below this many FLOPs take the fused kernel; larger ones expand the weight with the
@@ -328,7 +332,7 @@ class MatMulNF4(torch.autograd.Function):
                      and fused_pays(xc.numel() // max(xc.shape[-1], 1), *state.shape))
         if ctx.fused:
             return nf4_linear_fwd(xc, [(packed, state)], [bias], out_dtype)[0]
-        w = expand.take(packed, compute)  # expanded with the rest of its decoder layer
+        w = expand.take(packed, compute, state)  # expanded with the rest of its decoder layer
         if w is None:
             w = dequantize_nf4(packed, state, compute)
         if out_dtype == torch.float32 and compute != torch.float32 and xc.is_cuda:
@@ -361,9 +365,10 @@ class MatMulNF4(torch.autograd.Function):
         if ctx.fused and ctx.x_dtype in (torch.float16, torch.float32):
             dx = nf4_linear_bwd([g], [(ctx.packed, ctx.state)], ctx.x_dtype)
             return dx, None, None, None, None, None, d_res
-        w = expand.take(ctx.packed, g.dtype)
-        if w is None:  # the first expansion of a layer's backward expands the layer's group
-            w = expand.backward_group(ctx.packed, g.dtype)
+        w = expand.take(ctx.packed, g.dtype, ctx.state)
+        if w is None and expand.backward_group(ctx.packed, g.dtype) is not None:
+            # the first expansion of a layer's backward: the layer's group, this weight among it
+            w = expand.take(ctx.packed, g.dtype, ctx.state)
         if w is None:
             w = dequantize_nf4(ctx.packed, ctx.state, g.dtype)
         return torch.matmul(g, w).to(ctx.x_dtype), None, None, None, None, None, d_res

@@ -53,3 +53,79 @@ def test_layer_without_nf4_projections_is_left_alone():
     hidden = torch.zeros(1, 3, 4)
     expand.expand_layer(layer, hidden)
     assert not expand._READY.get(hidden.device.index)
+
+
+class State:
+    def __init__(self):
+        self.absmax = torch.zeros(1)
+
+
+def _left(*keys_pairs):
+    left = expand._Left(torch.device("cpu"))
+    for key, pairs in keys_pairs:
+        left.leave(key, torch.ones(2, 2, dtype=torch.float16), pairs)
+    expand._READY[None] = left
+    return left
+
+
+def test_take_rows_is_handed_out_once_in_its_order():
+    q, k, v = ((torch.zeros(8, dtype=torch.uint8), State()) for _ in range(3))
+    key = expand._rows_key([q[0], k[0], v[0]])
+    try:
+        w = _left((key, [q, k, v]))[key][0]
+        assert expand.take_rows([k, q, v]) is None  # the order of the stacked rows
+        assert expand.take_rows([q, k, v]) is w
+        assert expand.take_rows([q, k, v]) is None  # once
+        _left((key, [q, k, v]))
+        expand.drop(q[0].device)
+        assert expand.take_rows([q, k, v]) is None  # dropped
+    finally:
+        expand.drop(q[0].device)
+
+
+def test_left_expansions_are_of_the_weights_as_they_are():
+    """Not handed out for a weight written to since, a replaced QuantState, or rewritten scales."""
+    def changed(write):
+        packed, state = torch.zeros(8, dtype=torch.uint8), State()
+        _left((packed.data_ptr(), [(packed, state)]))
+        try:
+            state = write(packed, state) or state
+            return expand.take(packed, torch.float16, state)
+        finally:
+            expand.drop(packed.device)
+
+    assert changed(lambda p, s: None) is not None
+    assert changed(lambda p, s: (p.add_(1), None)[1]) is None
+    assert changed(lambda p, s: State()) is None
+    assert changed(lambda p, s: (s.absmax.add_(1), None)[1]) is None
+
+
+def test_left_expansions_end_with_their_backward():
+    """What a backward pass leaves is not handed out after it, nor in another one."""
+    packed, state = torch.zeros(8, dtype=torch.uint8), State()
+    seen = []
+
+    class Leaves(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, leave):
+            ctx.leave = leave
+            return x * 1
+
+        @staticmethod
+        def backward(ctx, g):
+            if ctx.leave:
+                _left((packed.data_ptr(), [(packed, state)]))
+            else:
+                seen.append(expand.take(packed, torch.float16, state))
+            return g, None
+
+    x = torch.ones(1, requires_grad=True)
+    try:
+        Leaves.apply(Leaves.apply(x, False), True).backward()
+        assert seen[0] is not None  # the same pass
+        Leaves.apply(x, True).backward()
+        assert expand.take(packed, torch.float16, state) is None  # after it
+        Leaves.apply(x, False).backward()
+        assert seen[1] is None  # another pass
+    finally:
+        expand.drop(packed.device)

@@ -24,17 +24,20 @@ using cm::gemm::KMajor;
 using cm::gemm::RowMajor;
 
 // Tiles of 256 x 192 on 4 x 2 wavefronts of 64 x 96: with four of 128 x 96 long slices take the same
-// time and short ones more (131 x 1536 x 17920 31 us against 27). With the sum, one MI355X:
-// 1276 x 1536 x 17920 97 -> 82 us, x 8960 58 -> 51 us (the loads spread over the main loop and no
-// bounds test for the partial row of tiles, gemm_lds.h).
+// time and short ones more (131 x 1536 x 17920 31 us against 27). With the sum, back to back in a graph,
+// one MI355X: 1276 x 1536 x 17920 91.5 -> 78.3 us, x 8960 53.6 -> 48.2 us; 130 tokens 36.7 -> 27.6, 23.9
+// -> 19.9; 300 tokens 38 -> 38.3, 26.3 -> 27.1 (the loads spread over the main loop and no bounds test for
+// the partial row of tiles, gemm_lds.h).
 constexpr int kBM = 256, kBN = 192, kWM = 4, kWN = 2, kBK = 64;
 constexpr int kSA = 3, kSB = 2;  // LDS stages of A and B: 144 KiB, one workgroup per CU
 constexpr int kThreads = kWM * kWN * cm::kWave;
 constexpr int kMaxSlices = 16;
 constexpr int kCUs = 256;
 
-// The fp32 partial tile of one K-slice, rows past M and columns past N dropped; with `residual` (the
-// one slice of an unsplit contraction), residual + the tile.
+// The fp32 partial tile of one K-slice, rows past M and columns past N dropped; with RES (the one slice
+// of an unsplit contraction), residual + the tile. RES is a kernel of its own: with a test of the
+// pointer beside each store the split kernels' epilogue doubled, 2.3 us of 22 at 130 x 1536 x 8960, 2.1 of 29 at 300.
+template <bool RES>
 struct EpiSlice {
   float* out;  // [M, N]: a slice of the workspace, or the result
   const float* residual;
@@ -59,9 +62,12 @@ struct EpiSlice {
 #pragma unroll
         for (int nt = 0; nt < TN; ++nt) {
           const int col = nb + nt * 32 + lane % 32;
-          if (col >= N) continue;
           const int64_t at = static_cast<int64_t>(row) * N + col;
-          out[at] = residual != nullptr ? residual[at] + acc[mt][nt][r] : acc[mt][nt][r];
+          if constexpr (RES) {
+            if (col < N) out[at] = residual[at] + acc[mt][nt][r];
+          } else {
+            if (col < N) out[at] = acc[mt][nt][r];
+          }
         }
       }
   }
@@ -74,7 +80,7 @@ struct Pairs {
   int k_slice[2];   // columns per slice of each pair (a multiple of 64)
 };
 
-template <bool KB>
+template <bool KB, bool RES>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int remap, float* ws,
                                                                const float* residual, int M,
                                                                int N) {
@@ -85,7 +91,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(Pairs p, int rema
   const int k_begin = sq * p.k_slice[q];
   // an empty slice still writes its (zero) partial tile, which the sum then reads
   const int k_end = max(k_begin, min(p.a[q].k_len, k_begin + p.k_slice[q]));
-  EpiSlice epi{ws + static_cast<int64_t>(s) * M * N, residual, M, N};
+  EpiSlice<RES> epi{ws + static_cast<int64_t>(s) * M * N, residual, M, N};
   if constexpr (KB) {
     if (q == 0) {
       cm::gemm::gemm_lds<kBM, kBN, kWM, kWN, kSA, kSB>(p.a[0], p.bk[0], k_begin, k_end, tm,
@@ -215,13 +221,11 @@ int gemm_f32_impl(const void* a0, int64_t lda0, const void* b0, int64_t ldb0, in
   hipStream_t s = static_cast<hipStream_t>(stream);
   float* ws = direct ? out : static_cast<float*>(workspace);
   const float* res = direct ? residual : nullptr;
-  if (b_kmajor) {
-    hipLaunchKernelGGL(gemm_f32_kernel<true>, dim3(tiles, pl.total()), dim3(kThreads), 0, s, p,
-                       remap, ws, res, M, N);
-  } else {
-    hipLaunchKernelGGL(gemm_f32_kernel<false>, dim3(tiles, pl.total()), dim3(kThreads), 0, s, p,
-                       remap, ws, res, M, N);
-  }
+  CM_CHECK_ARG(!(b_kmajor && residual));  // no entry point asks for both
+  const auto kernel = b_kmajor ? gemm_f32_kernel<true, false>
+                      : res    ? gemm_f32_kernel<false, true>
+                               : gemm_f32_kernel<false, false>;
+  hipLaunchKernelGGL(kernel, dim3(tiles, pl.total()), dim3(kThreads), 0, s, p, remap, ws, res, M, N);
   if (direct) return cm::launch_status();
   const int64_t n4 = static_cast<int64_t>(M) * N / 4;
   hipLaunchKernelGGL(gemm_f32_sum, dim3(static_cast<unsigned>((n4 + 255) / 256)), dim3(256), 0, s,

@@ -9,17 +9,32 @@ import pytest
 import torch
 
 # rows around the 64-, 128- and 256-row tiles; outputs that end inside a tile, one to three of them;
-# contractions from one stage; 8200 rows x 2048 take the 256 x 256 tiles, 2000 the 128 x 128 ones
+# contractions from one stage; with the tiles each way takes: 128 x 64 while one round of 256
+# workgroups holds the output, 256 x 256 (5400 rows, partial tiles both ways and along the contraction)
+# where its rounds are a third of 128 x 128's, else 128 x 128
 SHAPES = [
-    (1, 64, (64,)),
-    (63, 128, (64, 64)),
-    (127, 192, (192, 64, 128)),
-    (129, 64, (320, 64)),
-    (257, 576, (896, 128, 128)),
-    (1276, 1536, (1536, 256, 256)),
-    (2000, 320, (1536, 256, 256)),
-    (8200, 256, (1536, 256, 256)),
+    (1, 64, (64,), "narrow", "narrow"),
+    (63, 128, (64, 64), "narrow", "narrow"),
+    (127, 192, (192, 64, 128), "narrow", "narrow"),
+    (129, 64, (320, 64), "narrow", "narrow"),
+    (257, 576, (896, 128, 128), "narrow", "narrow"),
+    (1276, 1536, (1536, 256, 256), "small", "narrow"),
+    (2000, 320, (1536, 256, 256), "small", "narrow"),
+    (8200, 256, (1536, 256, 256), "small", "small"),
+    (5400, 1600, (1536, 192, 192), "large", "large"),
+    (5377, 1536, (1536, 256, 256), "large", "large"),
+    (4097, 1536, (1536, 256, 256), "large", "small"),
 ]
+
+
+def _form(m, n):
+    """The tiles cm_linear_f16_* takes for m x n outputs (launch_best in csrc/gemm_f16.hip)."""
+    def rounds(bm, bn):
+        return -(-(-(-m // bm) * -(-n // bn)) // 256)
+
+    if rounds(128, 64) <= 1:
+        return "narrow"
+    return "large" if rounds(256, 256) * 3 <= rounds(128, 128) else "small"
 
 
 def _bound(a, b, ref):
@@ -30,10 +45,11 @@ def _bound(a, b, ref):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,k,sizes", SHAPES)
-def test_linear_rows(dev, m, k, sizes):
+@pytest.mark.parametrize("m,k,sizes,fwd,bwd", SHAPES, ids=lambda v: str(v))
+def test_linear_rows(dev, m, k, sizes, fwd, bwd):
     from claudemaxing_amd.nf4_linear import linear_rows_bwd, linear_rows_fwd
 
+    assert (_form(m, sum(sizes)), _form(m, k)) == (fwd, bwd)
     g = torch.Generator(device=dev).manual_seed(m)
 
     def normal(*shape):

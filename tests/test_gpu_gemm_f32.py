@@ -123,12 +123,13 @@ def test_kmajor_b_row_stride(dev):
     assert not gemm_f32_supported(96, 60, (a, b[:, :60]), b_kmajor=True)  # N % 8
 
 
-@pytest.mark.parametrize("m,n,k0,k1", [(4096, 1536, 4104, 4104), (6001, 1544, 4096, 0), (255, 200, 64, 0),
-                                       (257, 8, 72, 0)])
-def test_one_slice_is_written_straight(m, n, k0, k1, dev):
-    """Contractions that are not split (enough tiles, or too few stages) go to the result without
-    partial sums: row-major and k-major B alike, with a residual too, edge tiles in m and n."""
-    banner(f"gemm_f32 unsplit m={m} n={n} k0={k0} k1={k1}")
+def _three_ways(m, n, k0, k1, slices, dev):
+    """Row-major and k-major B and, with a residual, the sum of both: against fp64, and each other's
+    bits; the workspace holds `slices` partial results."""
+    from claudemaxing_amd import _lib
+
+    banner(f"gemm_f32 {slices} slices m={m} n={n} k0={k0} k1={k1}")
+    assert _lib.load().cm_gemm_f32_workspace_bytes(m, n, k0, k1) == slices * 4 * m * n
     ref, rm, kb = 0, [], []
     for i, k in enumerate((k0, k1)):
         if k:
@@ -138,7 +139,22 @@ def test_one_slice_is_written_straight(m, n, k0, k1, dev):
             ref = ref + a.double() @ bt.t().double()
     out = gemm_f32(*rm)
     torch.cuda.synchronize()
-    _check(out, ref, "unsplit")
+    _check(out, ref, f"{slices} slices")
     assert torch.equal(out, gemm_f32(*kb, b_kmajor=True))
     res = torch.randn(m, n, device=dev, generator=torch.Generator(device=dev).manual_seed(13))
     assert torch.equal(gemm_f32(*rm, residual=res), res + out)
+
+
+@pytest.mark.parametrize("m,n,k0", [(4353, 1536, 4104), (6001, 1544, 4096), (255, 200, 64),
+                                    (256, 192, 64), (257, 8, 56)])
+def test_one_slice_is_written_straight(m, n, k0, dev):
+    """One pair that is not split (more than 128 tiles, or a single stage) goes to the result without
+    partial sums: row-major and k-major B alike, with a residual too, edges in m, n and k."""
+    _three_ways(m, n, k0, 0, 1, dev)
+
+
+@pytest.mark.parametrize("m,n,k0,k1", [(4096, 1536, 4104, 4104), (257, 8, 72, 0)])
+def test_two_slices(m, n, k0, k1, dev):
+    """The fewest that are summed: two pairs of one slice each (a second pair always has its own), and
+    one pair of two stages."""
+    _three_ways(m, n, k0, k1, 2, dev)

@@ -1,4 +1,4 @@
-"""NF4QKV (the q/k/v projections as one NF4-fused GEMM each way) against the three separate
+"""NF4QKV (the q/k/v projections as one GEMM on their expanded weights each way) against the three separate
 layers it replaces (LoRALinear over NF4Linear for q and v, NF4Linear for k), both held against an
 fp32 evaluation with the same dropout masks."""
 

@@ -72,8 +72,11 @@ constexpr int kThreads1 = kWM1 * kWN1 * cm::kWave;
 // 64 x 128 where it is a multiple of 256 (2048, 3584, 5120, 8192), else the first. The square
 // tile's rings stay at two stages of each operand: a third stage of E would leave no LDS for the
 // scales. Whole calls, one MI355X: N = 2048 at 1536 2102 -> 1950 us (four or eight wavefronts
-// alike), at 2048 2661 -> 2558 us (2575 on 2 x 4 wavefronts, 3181 on four, which spill, 3125 on
-// 256 x 192 tiles with a partial last one); 131 tokens at 1536 325 -> 292 us.
+// alike), at 2048 2661 -> 2558 us (2575 on 2 x 4 wavefronts, 3181 on four, which spill in the loop,
+// 3125 on 256 x 192 tiles with a partial last one); 131 tokens at 1536 325 -> 292 us. The kept square
+// tile spills as well (102-107 registers, 360-372 bytes of scratch per lane): its steady loop is free
+// of it, but the loads of the first stage each follow a reload and the first two stages reload
+// throughout.
 template <int BM, int BN, int WM, int WN, int SA, int SB, int OCC>
 struct K3Cfg {
   static constexpr int kBM = BM, kBN = BN, kWM = WM, kWN = WN, kSA = SA, kSB = SB, kOcc = OCC;
@@ -1115,6 +1118,8 @@ bool scratch_layout(int64_t n_rows, int64_t vocab, int hidden, int64_t chunk_col
     for (int64_t chunk = largest; chunk >= smallest; chunk -= kChunkAlign) {
       const Layout T = layout(n_rows, vocab, hidden, chunk, want_grad, sp);
       if (T.n_split < sp) continue;  // the same layout as a smaller count, visited later
+      // a smaller chunk's groups may split into more slices, whose accumulators take more
+      if (T.total > kScratchBytes) continue;
       any = true;
       const double cost = est_cost_us(n_rows, vocab, hidden, T);
       if (best_split == 0 || cost < best_cost) {
@@ -1127,7 +1132,7 @@ bool scratch_layout(int64_t n_rows, int64_t vocab, int hidden, int64_t chunk_col
   }
   if (best_split == 0) return false;
   *out = layout(n_rows, vocab, hidden, best_chunk, want_grad, best_split);
-  return out->total <= kScratchBytes;
+  return true;
 }
 
 }  // namespace

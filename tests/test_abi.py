@@ -295,3 +295,17 @@ def test_lmhead_plans(lib):
             groups = chunk // 128
             width = -(-groups // split)
             assert -(-groups // width) == split, (n, c, noalloc, chunk, split)
+
+
+@pytest.mark.parametrize("hidden", [896, 1536, 2048, 3584])
+def test_noalloc_plan_refuses_only_what_does_not_fit(lib, hidden):
+    """With its own chunk the no-allocation entry takes every batch that fits its scratch in
+    256-column chunks (K-slices and chunk trade off: a smaller chunk may split into more slices,
+    whose accumulators take more than its buffers save)."""
+    plan = lib.cm_lmhead_ce_noalloc_plan
+    chunk, split = ctypes.c_int64(), ctypes.c_int()
+    out = ctypes.byref(chunk), ctypes.byref(split)
+    for n in [*range(1, 1100), 2048, 5000, 16384]:
+        if plan(n, 151936, hidden, 256, 1, *out) == 0:
+            assert plan(n, 151936, hidden, 0, 1, *out) == 0, n
+            assert plan(n, 151936, hidden, chunk.value, 1, *out) == 0, n  # and it fits

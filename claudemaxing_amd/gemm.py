@@ -27,15 +27,20 @@ def split_k_pays(m, n, k):
 def kmajor_pays(m, n, k):
     """Whether an fp32-output product with a k-major weight (dx = y W) is worth the split-K GEMM: where
     split_k_pays, and on larger outputs while its tiles and slices fill one round of the 256 CUs to
-    nearly three quarters. There the product itself takes about the library's time, and what pays is
-    the merged weight it allows: one gate/up product along rows instead of two against transposed
-    copies. 1536 x 8960 MLP, recomputation + dx, us, merged / transposed: 4096 tokens (128 tiles x 2)
-    408 / 498, 6144 (192) 621 / 652, 8192 (256) 778 / 823; 5000 (160 tiles, 63%) 565 / 536; 2500
-    tokens of 3584 x 18944 (190) 1310 / 1775."""
+    nearly three quarters and its last column of tiles pads n by 2% at most. There the product itself
+    takes about the library's time, and what pays is the merged weight it allows: one gate/up product
+    along rows instead of two against transposed copies. MLP forward and backward, us, merged /
+    transposed: 1536 x 8960 at 4096 tokens (128 tiles x 2) 1073 / 1221, 5000 (160 tiles, 63%) 1355 /
+    1323, 5900 (192) 1460 / 1534, 6700 1673 / 1676, 8192 (256) 1880 / 1926, 9000 (288) 2259 / 2095;
+    3584 x 18944 at 2500 (190) 3096 / 3836, 3300 (247) 3686 / 3841. 2048 columns are 10.67 tiles, 3%
+    of padding, and gain at some sizes only: 2048 x 11008 at 4400 (198) 1845 / 1778, 4800 1929 / 2087,
+    5000 1934 / 1925, 5300 (231) 2099 / 2054."""
     if split_k_pays(m, n, k):
         return True
-    tiles = -(-m // 256) * -(-n // 192)
-    return k >= 4096 and tiles <= 256 and tiles * (256 // tiles) >= 184
+    cols = -(-n // 192)
+    tiles = -(-m // 256) * cols
+    return (k >= 4096 and tiles <= 256 and tiles * (256 // tiles) >= 184
+            and 50 * n >= 49 * 192 * cols)
 
 
 def gemm_f32_supported(m, n, *pairs, b_kmajor=False):

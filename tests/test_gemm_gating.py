@@ -26,6 +26,14 @@ def test_kmajor_pays_where_tiles_and_slices_fill_a_round():
     assert not kmajor_pays(8192, 1536, 1536)  # a short contraction
 
 
+def test_kmajor_pays_without_a_padded_column_of_tiles():
+    # 2048 columns are 10.67 tiles: past the narrow outputs the transposed copies are as fast or faster
+    for tokens in (4400, 5000, 5300):
+        assert not kmajor_pays(tokens, 2048, 2 * 11008), tokens
+    assert kmajor_pays(2500, 2048, 2 * 11008)  # as split_k_pays: 110 tiles
+    assert kmajor_pays(2500, 3584, 2 * 18944)  # 18.67 tiles, 1.8% of padding
+
+
 def test_cpu_operands_are_not_taken():
     a = torch.zeros(16, 64, dtype=torch.float16)
     b = torch.zeros(16, 64, dtype=torch.float16)

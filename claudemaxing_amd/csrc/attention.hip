@@ -402,12 +402,13 @@ __global__ __launch_bounds__(256) void attn_relayout_kernel(Jobs jobs, const Row
 // (one barrier each).
 //
 // What bounds them: below a few thousand tokens the serial chain of a block (at most one workgroup
-// per CU), above it the waits inside an iteration (fragment reads, softmax, barrier), which only the
-// SIMD's other wavefront covers: at 8191 tokens in one row, 12 heads, the backward's MFMAs take 35%
-// of the time. Backward with its relayout and head sum, one MI355X, before (one workgroup per CU,
-// transposed tiles) and now, same bits: 8191 tokens 1510 -> 995 us, 16 x 300 141 -> 108, 2048 + 1000
-// 174 -> 123, 4 rows of 154-482 51.6 -> 45.6. One pair per workgroup (four to a CU) was measured and
-// not kept: 2 x 4000 tokens 753 us against 813, but 2048 + 1000 164 against 125.
+// per CU), above it the waits inside an iteration (fragment reads, softmax, barrier, in the dK/dV
+// blocks the next tile's loads, see attn_bwd_kernel), which only the SIMD's other wavefront covers: at
+// 8191 tokens in one row, 12 heads, the backward's MFMAs take 34% of the time (40% of its busy CUs').
+// Backward with its relayout and head sum, one MI355X, before (one workgroup per CU, transposed tiles)
+// and now, same bits: 8191 tokens 1510 -> 995 us, 16 x 300 141 -> 108, 2048 + 1000 174 -> 123, 4 rows
+// of 154-482 51.6 -> 45.6. One pair per workgroup (four to a CU) was measured and not kept: 2 x 4000
+// tokens 753 us against 813, but 2048 + 1000 164 against 125.
 
 // Forward. Two forms, both with 32 queries per wavefront:
 //  - SPLIT: block (b, h) is 64 queries of one row, query head h (key/value head h / hpg); pair p
@@ -898,7 +899,10 @@ __device__ __forceinline__ void bwd_dq_block(const BwdArgs& a, int h, int b, uin
 constexpr int kBwdLds = 4 * (kDkdvStage > kDqStage ? kDkdvStage : kDqStage);
 
 // The LDS holds both pairs' double buffers (65 KiB: two workgroups per CU, so that one's softmax
-// and LDS waits run beside the other's MFMAs).
+// and LDS waits run beside the other's MFMAs). Two workgroups leave a wavefront 256 registers, 16 fewer
+// than the dK/dV blocks need: their loop reloads three 16-byte fragments from scratch, after the next
+// tile's direct loads were issued, and as both return in order the iteration's first MFMAs wait for
+// those too.
 template <typename OT>
 __global__ __launch_bounds__(kThreads, 2) void attn_bwd_kernel(BwdArgs a) {
   __shared__ uint4 raw[kBwdLds];

@@ -5,13 +5,14 @@
 // with fp32 sums, rounded once. The forward reads the weight by rows, the backward as stored, k-major
 // (its contraction runs over the weight rows), through transposing LDS reads (gemm_lds.h).
 //
-// What bounds it: at a training step's 1276 tokens the outputs are 160 tiles of 128 x 128 (forward)
-// or 120 (backward) on 256 CUs, each a serial chain of 24 to 32 stages of 64 columns that take ~0.25
-// us of matrix-core time: latency, so the loads run two stages ahead and the fragments most of a stage
-// (gemm_lds_small). Measured against the weights expanded inside the GEMM (nf4_gemm.hip, with its sum
-// over contraction slices), q/k/v of 1536 -> 1536 + 256 + 256, us forward / backward, the expansion
-// of the three weights (~5 us alone, less among a layer's others) not counted: 65 tokens 8.8 / 12.8
-// against 28 / 21; 1276 15.1 / 15 against 30 / 35; 8192 52 / 56 against 90 / 115.
+// What bounds it: at a training step's 1276 tokens the outputs are 160 tiles of 128 x 128 (forward,
+// contractions of 24 stages of 64 columns) or 240 of 128 x 64 (backward, 32 stages) on 256 CUs, one
+// workgroup each (the rings take 128 and 96 KiB of a CU's LDS), each a serial chain of stages that take
+// ~0.25 us of matrix-core time: latency, so the loads run two stages ahead and the fragments most of a
+// stage (gemm_lds_small). Measured against the weights expanded inside the GEMM (nf4_gemm.hip), q/k/v
+// of 1536 -> 1536 + 256 + 256, us forward / backward, the expansion of the three weights (~5 us alone,
+// less among a layer's others) not counted: 65 tokens 8.8 / 14.0 against 28 / 21; 1276 15.1 / 16.4
+// against 30 / 35; 8192 (256 x 256 tiles) 52 / 56 against 90 / 115.
 #include "gemm_lds.h"
 #include "nf4_tiles.h"
 

@@ -32,6 +32,7 @@ def test_kmajor_pays_without_a_padded_column_of_tiles():
         assert not kmajor_pays(tokens, 2048, 2 * 11008), tokens
     assert kmajor_pays(2500, 2048, 2 * 11008)  # as split_k_pays: 110 tiles
     assert kmajor_pays(2500, 3584, 2 * 18944)  # 18.67 tiles, 1.8% of padding
+    assert kmajor_pays(5883, 1600, 2 * 8960)  # 8.33 tiles, but 6.25 of the library's
 
 
 def test_cpu_operands_are_not_taken():

@@ -2,14 +2,14 @@
 
 python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--only NAME[,NAME...]]
 
-Every kernel runs on inputs already resident in HBM, at the shapes of BASELINE.json's configs:
+Every kernel runs on inputs already resident in HBM, at the headline configurations' shapes:
   1  NF4 dequant of the [8960,1536] gate_proj weight (blocksize 64, double-quantized) to fp16
   2  RMSNorm fwd/bwd and RoPE fwd/bwd on 4 packed rows of U[128,512] tokens (hidden 1536)
   3  SwiGLU forward and in-place recompute-backward on [2048,8960] fp16
   4  fused LM head + cross-entropy, hidden [2048,1536], tied weight [151936,1536] fp16
 plus the LoRA mask pack/unpack at the q/v input shape of config 5, every streaming kernel at a
 bandwidth-scale shape (32768 tokens; NF4 over one decoder layer's weights), the launch floor of
-the box (an empty kernel, a one-wavefront kernel, a 1 MiB copy), torch's device copy as the
+the machine (an empty kernel, a one-wavefront kernel, a 1 MiB copy), torch's device copy as the
 practical HBM ceiling, and config 5's QLoRA training step (eager over distinct batches, and
 replayed from a HIP graph).
 
@@ -64,7 +64,7 @@ def parse():
                    help="run the QLoRA step bench alone in this process and print its record as "
                         "one JSON line (what the default run starts as a child process)")
     p.add_argument("--no-peaks", action="store_true",
-                   help="skip the on-box HBM and matrix-core peak probes")
+                   help="skip the on-device HBM and matrix-core peak probes")
     p.add_argument("--no-power", action="store_true",
                    help="skip the board power sample of the headline (profiler runs)")
     return p.parse_args()
@@ -370,7 +370,7 @@ def k_copy_ref(dev):
 
 
 def k_floor(dev, names):
-    """What a launch costs on this box whatever it does: the library's empty kernel
+    """What a launch costs on this machine whatever it does: the library's empty kernel
     (cm_probe_launch, through the same ctypes path as every kernel here) with one wavefront and
     with the grid of the config-2 RoPE launch (1193 workgroups of 256 lanes), a one-wavefront
     torch kernel (a 64-element fill) and a 1 MiB torch device copy. The HIP-event figures here
@@ -1170,7 +1170,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "fp16" if headline == "lmhead_ce" else "u8->fp16",
-        "data": "synthetic (seeded CPU draws of BASELINE.json configs, copied to HBM)",
+        "data": "synthetic (seeded CPU draws of the headline configurations, copied to HBM)",
         "config": {"workload": headline, "shape": hr["config"], "parallelism": "none (1 GPU)",
                    "cold_cache": "input copies rotated beyond 512 MiB", **hr.get("plan", {})},
         "roofline": {"bound": hr["bound"], "achieved": hr["achieved"],

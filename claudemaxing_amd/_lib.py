@@ -174,7 +174,7 @@ def ptr(t):
 
 # torch's C accessor of the current stream's raw handle (what torch.cuda.current_stream(d)
 # .cuda_stream returns, without building a Stream object: 0.07 us against 1.9 us per call on the
-# MI355X box's host, and every launch asks for it); the public call where it is absent
+# MI355X's host, and every launch asks for it); the public call where it is absent
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 

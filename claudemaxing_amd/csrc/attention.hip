@@ -242,7 +242,7 @@ __device__ __forceinline__ half8 frag(const uint4* tile, int row, int c) {
 // rows are d = d0 .. d0 + 31: lane l gets d = d0 + l % 32 at positions 16 j + 4 h + 0 .. 3 and
 // 16 j + 8 + 4 h + 0 .. 3, h = l / 32. One ds_read_b64_tr_b16 each: lane a of a 16-lane group g
 // addresses 4 values of d at position k0 + a / 4 and receives positions k0 .. k0 + 3 of its own d
-// (lane layout checked on the box, gemm_lds.h).
+// (lane layout as in gemm_lds.h).
 __device__ __forceinline__ half8 frag_t(const uint4* tile, int d0, int j, int lane) {
   using cm::gemm::lds_short4_t;
   using cm::gemm::short4v;

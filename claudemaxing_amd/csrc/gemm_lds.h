@@ -247,7 +247,7 @@ typedef __attribute__((address_space(3))) short4v lds_short4_t;
 
 // The B fragment of v_mfma_f32_32x32x16_f16 (lane l: n = l % 32 of the 32-column tile at n_base,
 // k = ks * 16 + (l / 32) * 8 .. + 7) from a k-major LDS tile of BN columns, as two
-// ds_read_b64_tr_b16. That instruction (lane layout checked on the box) gives lane i of each
+// ds_read_b64_tr_b16. That instruction (lane layout checked by a probe kernel) gives lane i of each
 // 16-lane group element i % 4 of the 8 bytes that lane 4 j + i / 4 of the group addressed, for
 // j = 0 .. 3: so lane a of group g addresses row k0 + a / 4, columns n_base + 16 (g % 2) +
 // 4 (a % 4) .. + 3, and lane i receives rows k0 .. k0 + 3 of column n_base + 16 (g % 2) + i.

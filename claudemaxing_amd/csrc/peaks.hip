@@ -1,4 +1,4 @@
-// On-box probes of the two roofline denominators (measurement only; no counterpart in the
+// On-device probes of the two roofline denominators (measurement only; no counterpart in the
 // reference): the HBM bandwidth a streaming kernel attains on this board, and the fp16
 // matrix-core rate of v_mfma_f32_32x32x16_f16 with register operands. bench.py reports both
 // beside the published peaks (8 TB/s, 2.5 PFLOP/s), which the board reaches only at its top

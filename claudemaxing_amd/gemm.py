@@ -29,14 +29,13 @@ def kmajor_pays(m, n, k):
     split_k_pays, and on larger outputs while its tiles and slices fill one round of the 256 CUs to
     nearly three quarters, but not where its last column of tiles pads n by more than 2% and the
     library's 256-wide tiles pad nothing. There the product itself takes about the library's time, and
-    what pays is the merged weight it allows: one gate/up product
-    along rows instead of two against transposed copies. MLP forward and backward, us, merged /
-    transposed: 1536 x 8960 at 4096 tokens (128 tiles x 2) 1073 / 1221, 5000 (160 tiles, 63%) 1355 /
-    1323, 5900 (192) 1460 / 1534, 6700 1673 / 1676, 8192 (256) 1880 / 1926, 9000 (288) 2259 / 2095;
-    3584 x 18944 at 2500 (190) 3096 / 3836, 3300 (247) 3686 / 3841. 2048 columns are 10.67 tiles, 3%
-    of padding, and gain at some sizes only: 2048 x 11008 at 4400 (198) 1845 / 1778, 4800 1929 / 2087,
-    5000 1934 / 1925, 5300 (231) 2099 / 2054; 896 x 4864
-    (4.67 tiles here, 3.5 there) at 10000 (200) 1038 / 1085."""
+    what pays is the merged weight it allows: one gate/up product along rows instead of two against
+    transposed copies. MLP forward and backward, us, merged / transposed: 1536 x 8960 at 4096 tokens
+    (128 tiles x 2) 1073 / 1221, 5000 (160 tiles, 63%) 1355 / 1323, 5900 (192) 1460 / 1534, 6700 1673 /
+    1676, 8192 (256) 1880 / 1926, 9000 (288) 2259 / 2095; 3584 x 18944 at 2500 (190) 3096 / 3836, 3300
+    (247) 3686 / 3841. 2048 columns are 10.67 tiles, 3% of padding, and gain at some sizes only: 2048 x
+    11008 at 4400 (198) 1845 / 1778, 4800 1929 / 2087, 5000 1934 / 1925, 5300 (231) 2099 / 2054. 896 x
+    4864 (4.67 tiles here, 3.5 there) at 10000 (200): 1038 / 1085."""
     if split_k_pays(m, n, k):
         return True
     cols = -(-n // 192)

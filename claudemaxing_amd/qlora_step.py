@@ -438,7 +438,7 @@ class VramPoller:
     as the reference's harness samples nvidia-smi's memory.used every 100 ms
     (harness/common.py:48-85). The figure is device-level, total minus free
     (torch.cuda.mem_get_info): every process on the device, the runtime's own allocations and
-    torch's cache, not only torch's allocated bytes (amd-smi on these boxes reports no per-device
+    torch's cache, not only torch's allocated bytes (amd-smi here reports no per-device
     use). `start` is the first sample, `peak` the largest."""
 
     def __init__(self, device=None, interval=0.1):

@@ -577,7 +577,7 @@ int cm_nf4_dequant_group(const cm_nf4_weight* w, int n_w, void* const* out, int 
  * i - 1's (the [sum rows, cols] operand of cm_linear_f16_fwd / _bwd for weights of one width). */
 int cm_nf4_expand_rows(const cm_nf4_weight* w, int n_w, void* out, int out_dtype, void* stream);
 
-/* ---- On-box peak probes (measurement only; no counterpart in the reference) ----------------
+/* ---- On-device peak probes (measurement only; no counterpart in the reference) ----------------
  * The roofline denominators as this board attains them, which bench.py reports beside the
  * published 8 TB/s and 2.5 PFLOP/s. Neither is part of the training step. */
 

@@ -1,6 +1,6 @@
 """Seeded CPU generators of the benchmark configurations -- test infrastructure only.
 
-The shapes and distributions are those of BASELINE.json's configs (Qwen2.5-1.5B sizes): NF4
+The shapes and distributions are those of the headline configurations (Qwen2.5-1.5B sizes): NF4
 weight [8960,1536] N(0,0.02) blocksize 64 double-quantized; 4 packed rows of U[128,512] tokens,
 hidden 1536, 12/2 heads of 128, theta 1e6; SwiGLU [2048,8960]; LM head hidden [2048,1536] and
 tied weight [151936,1536] with 10% ignored labels. Everything is drawn on the CPU with

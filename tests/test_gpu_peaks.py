@@ -1,4 +1,4 @@
-"""The on-box peak probes bench.py reports beside the published peaks: the HBM stream copies
+"""The on-device peak probes bench.py reports beside the published peaks: the HBM stream copies
 exactly, the read-only stream and every matrix-core variant run, and the probe's FLOP count is
 the MFMAs it issues."""
 
